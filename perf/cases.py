@@ -10,7 +10,7 @@ Two paths are covered.
   (Q/K/V, gate and up) go in one call, as the decoder calls them.
 * "decoder": ``Decoder`` over a few layers of the package's TinyLlama-shaped
   configuration (``synth.TINYLLAMA``), or of the same width with wider heads:
-  prompts of 1 to 3072 tokens fed whole or in chunks, then decode steps, each
+  prompts of 2 to 2048 tokens fed whole or in chunks, then decode steps, each
   returning its logits; and greedy generation followed by one more forward.
 
 The package's contract is that every product and every logit has the bits of
