@@ -1,0 +1,566 @@
+// attention.hip -- causal attention of a prompt on gfx950's f32 matrix cores,
+// with the bits of the CPU path
+// (crates/rusticide-transformer/src/attention.rs:41-57,189-207,
+//  crates/rusticide-simd/src/float.rs:23-62,
+//  crates/rusticide-kernels/src/portable/norm.rs:17-30).
+//
+// The CPU path's order of float operations fits the f32 MFMA: one
+// v_mfma_f32_16x16x4 adds its four products to the accumulator one fused
+// multiply-add at a time, k ascending, each rounded to nearest with
+// subnormals kept (compared bit for bit with fmaf chains over normal,
+// subnormal, overflowing, signed-zero, infinite and NaN operands).
+//   * A score is eight interleaved chains of fused adds (dot's eight lanes),
+//     added in order: chain l is an accumulator of its own, its k the
+//     eight-wide chunks; the eight accumulators are then added in order.
+//   * An output lane's value mix is one chain over the rows: k is the row.
+#include <algorithm>
+#include <cmath>
+
+#include "rh_device.h"
+#include "rh_internal.h"
+#include "rh_math.h"
+
+namespace rh {
+
+namespace {
+
+constexpr uint32_t kStripQ = 16;       // (token, head) query rows a workgroup owns
+constexpr uint32_t kStripWaves = 8;
+constexpr uint32_t kStripThreads = 64u * kStripWaves;
+constexpr size_t kLdsBytes = 160u * 1024u;  // a gfx950 workgroup's LDS
+constexpr uint32_t kSumRounds = 6;     // checking rounds of the ordered sum
+
+constexpr int kBufferRsrcWord3 = 0x00020000;  // gfx9 buffer resource: raw 32-bit dwords
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+// A strip row holds one query row's scores, then its weights: four 16-byte
+// slots per group of 16 cached rows, slot 4 group + kr holding rows 4i + kr,
+// i = 0..3, of the group -- the four k of an MFMA step side by side across
+// the lanes that read them, four steps a read. The slots of 16 are exchanged
+// by their position so that lanes reading runs of a row, one run a lane,
+// fall on distinct banks; the row's length (an odd number of slots) does the
+// same for lanes reading one slot of 16 rows.
+__device__ __forceinline__ uint32_t strip_slot(uint32_t f4) { return f4 ^ ((f4 >> 4) & 15u); }
+
+__host__ __device__ constexpr uint32_t strip_stride(uint32_t groups) { return 16u * ((groups + 3u) & ~3u) + 4u; }
+
+constexpr size_t strip_lds_bytes(uint32_t groups) {
+  // strip | per-wave maxima [waves][16] | the exp table
+  return 4u * (static_cast<size_t>(kStripQ) * strip_stride(groups) + kStripWaves * kStripQ) + 32u * 8u;
+}
+
+// x[i] / d, given inv = 1 / d in double, correctly rounded. The double
+// quotient is within 2^-52 of x / d relatively; a quotient of two floats is
+// never closer than 2^-49 to the midpoint of two normal floats, so rounding
+// it gives the float nearest x / d. Subnormal midpoints have fewer bits and
+// a quotient may be one: where the result is subnormal the division itself
+// is taken (one branch for the four). A midpoint at the ends of that range,
+// 2^-150 and 2^-126 - 2^-150, rounds out of it (to even), and the quotient
+// that lands inside it by its error is among those divided.
+template <typename V>
+__device__ __forceinline__ void div_by(V& x, float d, double inv) {
+  constexpr int kSubnormal = 0x90;  // v_cmp_class: subnormal of either sign
+  float q[4];
+  bool sub = false;
+#pragma unroll
+  for (uint32_t i = 0; i < 4u; i++) {
+    q[i] = static_cast<float>(static_cast<double>(x[i]) * inv);
+    sub |= __builtin_amdgcn_classf(q[i], kSubnormal);
+  }
+  if (sub) {
+#pragma unroll
+    for (uint32_t i = 0; i < 4u; i++) q[i] = __fdiv_rn(x[i], d);
+  }
+#pragma unroll
+  for (uint32_t i = 0; i < 4u; i++) x[i] = q[i];
+}
+
+// Inclusive prefix sum over each half of the wave (approximate: guesses).
+__device__ __forceinline__ double half_prefix_sum(double v) {
+  v += dpp_fill0_f64<0x111>(v);
+  v += dpp_fill0_f64<0x112>(v);
+  v += dpp_fill0_f64<0x114>(v);
+  v += dpp_fill0_f64<0x118>(v);
+  v += dpp_fill0_f64<0x142, 0xA>(v);
+  return v;
+}
+
+// Start guesses from increments, per half-wave: its first lane gets 0, lane
+// k the increments of the lanes before it.
+__device__ __forceinline__ float half_guess_starts(double d, uint32_t hl) {
+  const float end = static_cast<float>(half_prefix_sum(d));
+  const uint32_t prev = dpp_fill<kDppWaveShr1>(__float_as_uint(end), 0u);
+  return __uint_as_float(hl == 0u ? 0u : prev);
+}
+
+__device__ __forceinline__ uint32_t half_prefix_maps_excl(uint32_t m, uint32_t hl) {
+  m = map_after(m, dpp_fill<0x111>(m, kMapIdentity));
+  m = map_after(m, dpp_fill<0x112>(m, kMapIdentity));
+  m = map_after(m, dpp_fill<0x114>(m, kMapIdentity));
+  m = map_after(m, dpp_fill<0x118>(m, kMapIdentity));
+  m = map_after(m, dpp_fill<0x142, 0xA>(m, kMapIdentity));
+  const uint32_t prev = dpp_fill<kDppWaveShr1>(m, kMapIdentity);
+  return hl == 0u ? kMapIdentity : prev;
+}
+
+// The 16 values of group gi of a strip row, in row order.
+__device__ __forceinline__ void load_group(const float* row, uint32_t gi, float (&x)[16]) {
+#pragma unroll
+  for (uint32_t kr = 0; kr < 4u; kr++) {
+    const f32x4 t = reinterpret_cast<const f32x4*>(row)[strip_slot(4u * gi + kr)];
+#pragma unroll
+    for (uint32_t i = 0; i < 4u; i++) x[4u * i + kr] = t[i];
+  }
+}
+
+// The sum in order from 0.0 of a strip row per half-wave (ordered_sum_wave's
+// method, rh_device.h, with 32 lanes a sum): lane hl holds the run of `mine`
+// groups from group hl * per on, `lanes` lanes hold values, and t is an
+// approximate sum of the lane's run. Every lane of the wave calls it.
+__device__ __forceinline__ float ordered_sum_half(const float* row, uint32_t per, uint32_t mine, uint32_t lanes,
+                                                  uint32_t groups, float t) {
+  const uint32_t lane = __lane_id(), hl = lane & 31u, half = lane >> 5;
+  const uint32_t g0 = hl * per;
+  double d = t;
+  {
+    const float g = half_guess_starts(d, hl);
+    float e = g;
+    for (uint32_t c = 0; c < mine; c++) {
+      float x[16];
+      load_group(row, g0 + c, x);
+#pragma unroll
+      for (int i = 0; i < 16; i++) e += x[i];
+    }
+    d = static_cast<double>(e) - static_cast<double>(g);
+  }
+  for (uint32_t r = 1;; r++) {
+    const float g = half_guess_starts(d, hl);
+    const uint32_t gb = __float_as_uint(g);
+    const float cand[3] = {g, __uint_as_float(gb - 1u), __uint_as_float(gb + 1u)};
+    float s[3] = {cand[0], cand[1], cand[2]};
+    for (uint32_t c = 0; c < mine; c++) {
+      float x[16];
+      load_group(row, g0 + c, x);
+#pragma unroll
+      for (int i = 0; i < 16; i++) {
+        s[0] += x[i];
+        s[1] += x[i];
+        s[2] += x[i];
+      }
+    }
+    uint32_t next = dpp_fill<kDppWaveShl1>(gb, 0u);
+    asm volatile("" : "+v"(next));  // kept out of DPP combining, as in ordered_sum_wave4
+    uint32_t map = 0x03000000u;
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+      const uint32_t delta = __float_as_uint(s[i]) - next;
+      const uint32_t neg = delta >> 31;
+      const uint32_t mag = min(neg ? 0u - delta : delta, 2u);
+      map |= min(2u * mag - neg, 3u) << (8 * i);
+    }
+    if (hl + 1u >= lanes) map = kMapIdentity;
+    const uint32_t state = half_prefix_maps_excl(map, hl) & 0xFFu;
+    const float mine_end = state == 1u ? s[1] : state == 2u ? s[2] : s[0];
+    const uint64_t bad = __ballot(hl < lanes && state == 3u);
+    const uint32_t bad_h = static_cast<uint32_t>(bad >> (32u * half));
+    const uint32_t fb = bad_h ? static_cast<uint32_t>(__builtin_ctz(bad_h)) : lanes;  // >= 1
+    if (bad == 0 || r == kSumRounds) {
+      float end = __shfl(mine_end, static_cast<int>(32u * half + fb - 1u), 64);
+      // unresolved runs of the last round are added one value at a time
+      for (uint32_t c = fb * per; c < groups; c++) {
+        float x[16];
+        load_group(row, c, x);
+#pragma unroll
+        for (int i = 0; i < 16; i++) end += x[i];
+      }
+      return end;
+    }
+    const float start = state == 1u ? cand[1] : state == 2u ? cand[2] : cand[0];
+    d = hl < fb ? static_cast<double>(mine_end) - static_cast<double>(start)
+                : static_cast<double>(s[0]) - static_cast<double>(cand[0]);
+  }
+}
+
+// The cached rows of one layer in the strips' operand order, a group of 16
+// rows at a time: consecutive lanes of an operand hold consecutive rows (keys)
+// or output lanes (values), which in row order lie apart, and a load whose
+// lanes lie apart costs a cycle a lane (the strips read every row once for
+// each 16 query rows: 256 tokens behind 1744 rows spent 15.6 us in the scores
+// and 13.8 in the mix on such loads).
+//   keys: [kv head][group][HD / 4 pieces of four values][operand row][4],
+//         operand row j being row 4 (j % 4) + j / 4 of the group;
+//   values: [kv head][group][HD / 16][k = row % 4][16 output lanes][row / 4].
+// cap: groups a kv head has room for.
+template <uint32_t HD>
+__global__ __launch_bounds__(256) void pack_kv_kernel(const float* __restrict__ kcache,
+                                                      const float* __restrict__ vcache, uint32_t kv, uint32_t rows,
+                                                      uint32_t cap, float* __restrict__ kpack,
+                                                      float* __restrict__ vpack) {
+  const uint32_t g = blockIdx.x, kvh = blockIdx.y, off = kvh * HD;
+  const size_t to = static_cast<size_t>(kvh * cap + g) * 16u * HD;
+#pragma unroll
+  for (uint32_t t = threadIdx.x; t < 4u * HD; t += 256u) {
+    const uint32_t e4 = t % (HD / 4u), rr = t / (HD / 4u), j = (rr & 3u) * 4u + (rr >> 2);
+    reinterpret_cast<f32x4*>(kpack + to)[16u * e4 + j] = *reinterpret_cast<const f32x4*>(
+        kcache + static_cast<size_t>(min(16u * g + rr, rows - 1u)) * kv + off + 4u * e4);
+    const uint32_t d = t % HD, kr = t / HD;
+    f32x4 x;
+#pragma unroll
+    for (uint32_t i = 0; i < 4u; i++)
+      x[i] = vcache[static_cast<size_t>(min(16u * g + 4u * i + kr, rows - 1u)) * kv + off + d];
+    reinterpret_cast<f32x4*>(vpack + to)[64u * (d >> 4) + 16u * kr + (d & 15u)] = x;
+  }
+}
+
+// A workgroup owns 16 query rows -- 16 >> hs_log tokens of (1 << hs_log)
+// heads that share a kv head -- over all their cached rows, three phases
+// apart by a barrier:
+//   1. scores: each wave takes groups of 16 cached rows in turn, HD / 4
+//      MFMAs a 16 x 16 tile, the keys straight from memory into the A operand;
+//   2. softmax: each half-wave takes one query row: exp, the ordered sum,
+//      the division, in LDS;
+//   3. the value mix: wave w owns output lanes 16w .. of all 16 query rows,
+//      one MFMA per four cached rows, values straight from memory. The groups that reach past some query row's last cached
+//      row are added lane by lane, so that no masked row enters a chain.
+// The scores stay in LDS between the phases (64 bytes a cached row), which
+// caps a launch at kStripMaxGroups groups.
+// What bounds it: the two products' MFMAs, HD / 4 of 32 cycles each a 16 x 16
+// tile on four SIMDs, 13 us of a strip over 2000 rows of 64; measured, the
+// scores take 9.7 us of it, the mix, one chain a SIMD, 11.9, and the softmax
+// between them, which one workgroup a CU cannot overlap, 13.
+// 2000 tokens of 32 heads of 64 over 4 kv heads: 339 us a layer with the
+// packing, against 2521 for attention_group_kernel (a workgroup a token and
+// kv head); 700 tokens of 16 heads of 128: 50 us against 381 for
+// attention_kernel.
+// ONE: one workgroup has the CU (strips over half its LDS), so a wave has
+// twice the registers, and keeps more of its loads in flight.
+template <uint32_t HD, bool ONE>
+__global__ __launch_bounds__(kStripThreads, !ONE && HD == 64u ? 4 : 2) void attention_strip_kernel(
+    const float* __restrict__ q, const float* __restrict__ kpack, const float* __restrict__ vpack,
+    const float* __restrict__ vcache, uint32_t cap, uint32_t width, uint32_t kv, uint32_t heads, uint32_t hs_log, uint32_t group, float scale, uint32_t start, uint32_t n,
+    uint32_t tile0, uint32_t tiles, uint32_t stride, float* __restrict__ mixed) {
+  constexpr uint32_t MQ = HD / 32u;   // MFMA steps of a score chain
+  constexpr uint32_t DT = HD / 16u;   // output tiles of 16 lanes
+  constexpr uint32_t KA = ONE ? 4u : 2u, kMixAhead = ONE ? 16u : 8u;  // groups of keys, of values requested ahead
+  static_assert(DT <= kStripWaves, "a wave an output tile");
+  extern __shared__ __align__(16) float sh[];
+  float* const strip = sh;                              // [16][stride]
+  float* const red = strip + kStripQ * stride;          // [waves][16]
+  uint64_t* const table = reinterpret_cast<uint64_t*>(red + kStripWaves * kStripQ);
+  const uint32_t tid = threadIdx.x, lane = tid & 63u;
+  const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(tid >> 6)));
+  const uint32_t j = lane & 15u, kq = lane >> 4;        // the lane's query row (or operand row) and k
+  const uint32_t tps = kStripQ >> hs_log;               // tokens a strip
+  // the longest strips first
+  const uint32_t hx = heads >> hs_log, ty = (blockIdx.x & 7u) + 8u * ((blockIdx.x >> 3) / hx);
+  if (ty >= tiles) return;
+  const uint32_t t0 = (tile0 + tiles - 1u - ty) * tps;
+  const uint32_t h0 = ((blockIdx.x >> 3) % hx) << hs_log, off = (h0 / group) * HD;
+  const uint32_t tj = t0 + (j >> hs_log), hj = h0 + (j & ((1u << hs_log) - 1u));
+  const uint32_t tc = min(tj, n - 1u);                  // past the batch: its last token, not stored
+  const uint32_t pos = start + tc;                      // the last cached row of query row j
+  const uint32_t last = start + min(t0 + tps - 1u, n - 1u);
+  const uint32_t groups = (last >> 4) + 1u, full = (start + t0 + 1u) >> 4;  // full: whole for every query row
+
+  if (tid < 32u) table[tid] = exp_table_entry(tid);
+
+  // ---- scores
+  // chain l, step m: k = kq is chunk c = 4m + kq, element 8c + l
+  const float* const qp = q + static_cast<size_t>(tc) * width + hj * HD + 8u * kq;
+  f32x4 qf[MQ][2];
+#pragma unroll
+  for (uint32_t m = 0; m < MQ; m++)
+#pragma unroll
+    for (uint32_t u = 0; u < 2u; u++) qf[m][u] = *reinterpret_cast<const f32x4*>(qp + 32u * m + 4u * u);
+  // the group's keys in operand order (pack_kv_kernel): D's registers i of
+  // lane (j, kq) are rows 4i + kq, a slot of the strip
+  const uint32_t pg = (h0 / group) * cap;  // the kv head's first packed group
+  const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(kpack + static_cast<size_t>(pg) * 16u * HD), 0, static_cast<int>(groups * 64u * HD),
+      kBufferRsrcWord3);
+  auto load_k = [&](f32x4 (&f)[MQ][2], uint32_t gi) {
+    const int base = static_cast<int>(min(gi, groups - 1u) * 64u * HD);
+#pragma unroll
+    for (uint32_t m = 0; m < MQ; m++)
+#pragma unroll
+      for (uint32_t u = 0; u < 2u; u++)
+        f[m][u] = __builtin_bit_cast(
+            f32x4, __builtin_amdgcn_raw_buffer_load_b128(krs, static_cast<int>(512u * kq + 16u * j),
+                                                         base + static_cast<int>(256u * (8u * m + u)), 0));
+  };
+  const double inv_scale = 1.0 / static_cast<double>(scale);
+  float mx = -INFINITY;
+  auto score = [&](const f32x4 (&f)[MQ][2], uint32_t gi) {
+    v4f acc[8];
+#pragma unroll
+    for (uint32_t m = 0; m < MQ; m++)
+#pragma unroll
+      for (uint32_t l = 0; l < 8u; l++)
+        acc[l] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[m][l >> 2][l & 3u], qf[m][l >> 2][l & 3u],
+                                                      m ? acc[l] : v4f{}, 0, 0, 0);
+    f32x4 sc;
+#pragma unroll
+    for (uint32_t i = 0; i < 4u; i++) {
+      float s = acc[0][i];
+#pragma unroll
+      for (uint32_t l = 1; l < 8u; l++) s += acc[l][i];
+      sc[i] = s;
+    }
+    // attention.rs:189-207: over sqrt(head_dim); 8 is a power of two
+    if constexpr (HD == 64u) sc *= 0.125f;
+    else div_by(sc, scale, inv_scale);
+    // past the query row's last cached row: -inf, which the maximum drops and
+    // whose exp, 0, changes no sum
+    if (gi >= full) {
+#pragma unroll
+      for (uint32_t i = 0; i < 4u; i++)
+        if (16u * gi + 4u * i + kq > pos) sc[i] = -INFINITY;
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < 4u; i++) mx = fmaxf(mx, sc[i]);
+    reinterpret_cast<f32x4*>(strip + j * stride)[strip_slot(4u * gi + kq)] = sc;
+  };
+  // KA register sets by turns, each requested again as soon as it is used (a
+  // copy between sets would wait for its loads)
+  f32x4 kf[KA][MQ][2];
+#pragma unroll
+  for (uint32_t a = 0; a < KA; a++) load_k(kf[a], wave + a * kStripWaves);
+  uint32_t gw = wave;
+  for (; gw + (KA - 1u) * kStripWaves < groups; gw += KA * kStripWaves) {
+#pragma unroll
+    for (uint32_t a = 0; a < KA; a++) {
+      score(kf[a], gw + a * kStripWaves);
+      load_k(kf[a], gw + (a + KA) * kStripWaves);
+    }
+  }
+#pragma unroll
+  for (uint32_t a = 0; a + 1u < KA; a++)
+    if (gw + a * kStripWaves < groups) score(kf[a], gw + a * kStripWaves);
+  mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+  if (lane < kStripQ) red[wave * kStripQ + lane] = mx;
+  __syncthreads();
+
+  // ---- softmax (norm.rs:17-30): half-wave `half` of each wave takes query row jr
+  {
+    static_assert(kStripQ == 2u * kStripWaves, "a query row a half-wave");
+    const uint32_t half = lane >> 5, hl = lane & 31u, jr = 2u * wave + half;
+    const uint32_t rows = start + min(t0 + (jr >> hs_log), n - 1u) + 1u;
+    float* const row = strip + jr * stride;
+    float m = red[jr];
+#pragma unroll
+    for (uint32_t w = 1; w < kStripWaves; w++) m = fmaxf(m, red[w * kStripQ + jr]);
+    const uint32_t per = (groups + 31u) >> 5;
+    const uint32_t own = (rows + 15u) >> 4, lanes = (own + per - 1u) / per;
+    const uint32_t mine = hl < lanes ? min(per, own - hl * per) : 0u;
+    float t = 0.0f;
+    for (uint32_t c = 0; c < mine; c++) {
+      const uint32_t gi = hl * per + c;
+#pragma unroll
+      for (uint32_t kr = 0; kr < 4u; kr++) {
+        f32x4* const at = reinterpret_cast<f32x4*>(row) + strip_slot(4u * gi + kr);
+        f32x4 x = *at;
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; i++) {
+          // x - max is at most 0, or NaN
+          const float d = x[i] - m, e = expf_ref_inner(d, [&](uint32_t k) { return table[k]; });
+          x[i] = d < -0x1.9fe368p6f ? 0.0f : e;
+        }
+        *at = x;
+        t += (x[0] + x[1]) + (x[2] + x[3]);
+      }
+    }
+    const float sum = ordered_sum_half(row, per, mine, lanes, own, t);
+    const double inv = 1.0 / static_cast<double>(sum);
+    for (uint32_t c = 0; c < mine; c++) {
+#pragma unroll
+      for (uint32_t kr = 0; kr < 4u; kr++) {
+        f32x4* const at = reinterpret_cast<f32x4*>(row) + strip_slot(4u * (hl * per + c) + kr);
+        f32x4 x = *at;
+        div_by(x, sum, inv);
+        *at = x;
+      }
+    }
+  }
+  __syncthreads();
+
+  // ---- value mix (float.rs:52-62): out starts at 0.0, each row fused in order
+  if (wave >= DT) return;
+  const f32x4* const wrow = reinterpret_cast<const f32x4*>(strip + j * stride);
+  v4f acc{};
+  if (full) {
+    const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(vpack + static_cast<size_t>(pg) * 16u * HD), 0, static_cast<int>(full * 64u * HD),
+        kBufferRsrcWord3);
+    f32x4 v[kMixAhead];
+    auto load_v = [&](f32x4& x, uint32_t gi) {
+      x = __builtin_bit_cast(
+          f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                     prs, static_cast<int>(16u * lane),
+                     static_cast<int>(min(gi, full - 1u) * 64u * HD + 1024u * wave), 0));
+    };
+    auto mix = [&](const f32x4& x, const f32x4& w) {
+#pragma unroll
+      for (uint32_t i = 0; i < 4u; i++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i], w[i], acc, 0, 0, 0);
+    };
+    auto weights = [&](uint32_t gi) { return wrow[strip_slot(4u * min(gi, full - 1u) + kq)]; };
+#pragma unroll
+    for (uint32_t a = 0; a < kMixAhead; a++) load_v(v[a], a);
+    f32x4 w[2] = {weights(0u), weights(1u)};
+    uint32_t g0 = 0;
+    // whole rounds of the register sets without a branch, so that the loads
+    // in flight are counted exactly at each wait
+    for (; g0 + kMixAhead <= full; g0 += kMixAhead) {
+#pragma unroll
+      for (uint32_t a = 0; a < kMixAhead; a++) {
+        mix(v[a], w[a & 1u]);
+        load_v(v[a], g0 + a + kMixAhead);
+        w[a & 1u] = weights(g0 + a + 2u);
+      }
+    }
+#pragma unroll
+    for (uint32_t a = 0; a + 1u < kMixAhead; a++)
+      if (g0 + a < full) {
+        mix(v[a], w[a & 1u]);
+        w[a & 1u] = weights(g0 + a + 2u);
+      }
+  }
+  // acc[i] is query row j's output lane 16 wave + 4 kq + i
+  const int kvb = static_cast<int>(4u * kv);
+  const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(vcache), 0, static_cast<int>(last + 1u) * kvb, kBufferRsrcWord3);
+  for (uint32_t gi = full; gi < groups; gi++) {
+    float w[16];
+    load_group(reinterpret_cast<const float*>(wrow), gi, w);
+#pragma unroll
+    for (uint32_t half = 0; half < 16u; half += 8u) {
+      f32x4 x[8];
+#pragma unroll
+      for (uint32_t r = 0; r < 8u; r++)
+        x[r] = __builtin_bit_cast(
+            f32x4, __builtin_amdgcn_raw_buffer_load_b128(vrs, static_cast<int>(4u * (off + 16u * wave + 4u * kq)),
+                                                         static_cast<int>(min(16u * gi + half + r, last)) * kvb, 0));
+#pragma unroll
+      for (uint32_t r = 0; r < 8u; r++)
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; i++) {
+          const float s = __builtin_fmaf(x[r][i], w[half + r], acc[i]);
+          acc[i] = 16u * gi + half + r <= pos ? s : acc[i];
+        }
+    }
+  }
+  if (tj < n)
+    *reinterpret_cast<f32x4*>(mixed + static_cast<size_t>(tj) * width + hj * HD + 16u * wave + 4u * kq) =
+        f32x4{acc[0], acc[1], acc[2], acc[3]};
+}
+
+// q/k/v from the projections, token-major: q and k rotated
+// (portable/rope.rs:7-23), k and v into the cache at positions start + t. One
+// thread per rotation pair (q, k) or pair of value elements.
+__global__ __launch_bounds__(256) void rope_append_kernel(const float* __restrict__ qr, const float* __restrict__ kr,
+                                                          const float* __restrict__ vr, uint32_t width, uint32_t kv,
+                                                          uint32_t head_dim, const float* __restrict__ rcos,
+                                                          const float* __restrict__ rsin, uint32_t start,
+                                                          float* __restrict__ q, float* __restrict__ kcache,
+                                                          float* __restrict__ vcache) {
+  const uint32_t t = blockIdx.y, i = blockIdx.x * 256u + threadIdx.x;
+  const uint32_t pos = start + t, qp = width / 2u, kp = kv / 2u;
+  if (i < qp + kp) {
+    const bool is_q = i < qp;
+    const uint32_t e = is_q ? i : i - qp, pairs = head_dim / 2u, p = e % pairs;
+    const f32x2 x = reinterpret_cast<const f32x2*>(is_q ? qr + static_cast<size_t>(t) * width
+                                                        : kr + static_cast<size_t>(t) * kv)[e];
+    const float c = rcos[static_cast<size_t>(pos) * pairs + p], s = rsin[static_cast<size_t>(pos) * pairs + p];
+    const float hs = x[1] * s, ls = x[0] * s;
+    f32x2 y;
+    y[0] = __builtin_fmaf(x[0], c, -hs);
+    y[1] = __builtin_fmaf(x[1], c, ls);
+    reinterpret_cast<f32x2*>(is_q ? q + static_cast<size_t>(t) * width : kcache + static_cast<size_t>(pos) * kv)[e] = y;
+  } else if (i < qp + 2u * kp) {
+    const uint32_t e = i - qp - kp;
+    reinterpret_cast<f32x2*>(vcache + static_cast<size_t>(pos) * kv)[e] =
+        reinterpret_cast<const f32x2*>(vr + static_cast<size_t>(t) * kv)[e];
+  }
+}
+
+// The most groups of a strip of which `fit` share a CU's LDS.
+constexpr uint32_t strip_max_groups(uint32_t fit) {
+  uint32_t g = 0;
+  while (strip_lds_bytes(g + 4u) * fit <= kLdsBytes) g += 4u;
+  return g;
+}
+constexpr uint32_t kStripMaxGroups = strip_max_groups(1u), kStripHalfGroups = strip_max_groups(2u);
+
+template <uint32_t HD>
+hipError_t launch_strips(const float* q, const float* kcache, const float* vcache, float* pack, uint32_t cap,
+                         uint32_t width, uint32_t kv, uint32_t heads, uint32_t group, float scale, uint32_t start,
+                         uint32_t n, float* mixed, hipStream_t s) {
+  float* const vpack = pack + static_cast<size_t>(cap) * 16u * kv;
+  hipLaunchKernelGGL((pack_kv_kernel<HD>), dim3((start + n + 15u) / 16u, kv / HD), dim3(256), 0, s, kcache, vcache, kv,
+                     start + n, cap, pack, vpack);
+  if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+  // heads a strip: the query heads of a kv head as far as 16 rows hold them
+  // evenly (the tokens of a strip then span few rows past the shared groups)
+  uint32_t hs_log = 0;
+  while (hs_log < 4u && group % (2u << hs_log) == 0) hs_log++;
+  const uint32_t tps = kStripQ >> hs_log, tiles = (n + tps - 1u) / tps;
+  // tokens whose strips take less than half the LDS go in a launch of their
+  // own, two workgroups a CU, where they have work for the whole chip
+  const uint32_t half = 16u * kStripHalfGroups;  // rows of those strips
+  uint32_t cut = half > start ? std::min(tiles, (half - start) / tps) : 0u;
+  if (cut < tiles && cut * (heads >> hs_log) < 512u) cut = 0;
+  for (uint32_t part = 0; part < 2u; part++) {
+    const uint32_t t0 = part ? cut : 0u, t1 = part ? tiles : cut;
+    if (t0 == t1) continue;
+    const uint32_t groups = (start + std::min(t1 * tps, n) - 1u) / 16u + 1u;
+    const auto fn = groups > kStripHalfGroups ? attention_strip_kernel<HD, true> : attention_strip_kernel<HD, false>;
+    hipLaunchKernelGGL(fn, dim3((heads >> hs_log) * ((t1 - t0 + 7u) & ~7u)), dim3(kStripThreads),
+                       strip_lds_bytes(groups), s, q, pack, vpack, vcache, cap, width, kv, heads, hs_log, group, scale,
+                       start, n, t0, t1 - t0, strip_stride(groups), mixed);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+}  // namespace
+
+// Rows from which strips are the faster where attention_group_kernel takes the
+// shape: it needs no packing, no RoPE and no quantize launch. Two layers of a
+// 64-token batch, wall clock, 32/4 heads of 64: 219 us against 222 at 192 rows,
+// 219 against 227 at 256, 227 against 261 at 512; 16 tokens: 203 against 200
+// at 208 rows, 205 against 211 at 272. Heads of 128 (attention_kernel) gain at
+// every length: 224 against 233 us at 64 rows.
+constexpr size_t kStripMinRows = 224;
+
+bool attention_strip_ok(size_t head_dim, size_t rows, size_t n, bool grouped) {
+  return (head_dim == 64u || head_dim == 128u) && rows <= 16u * kStripMaxGroups && n >= 2u &&
+         (!grouped || rows >= kStripMinRows);
+}
+
+// Groups a kv head has room for in the packed rows, and their floats.
+static uint32_t strip_cap(size_t context) {
+  return static_cast<uint32_t>(std::min<size_t>((context + 15u) / 16u, kStripMaxGroups));
+}
+size_t attention_pack_floats(size_t context, size_t kv) { return 2u * strip_cap(context) * size_t{16} * kv; }
+
+hipError_t launch_attention_strip(const float* q, const float* kcache, const float* vcache, float* pack,
+                                  size_t context, uint32_t width, uint32_t kv, uint32_t head_dim, float scale,
+                                  uint32_t start, uint32_t n, float* mixed, hipStream_t s) {
+  const uint32_t heads = width / head_dim, group = heads / (kv / head_dim), cap = strip_cap(context);
+  if (head_dim == 64u)
+    return launch_strips<64>(q, kcache, vcache, pack, cap, width, kv, heads, group, scale, start, n, mixed, s);
+  return launch_strips<128>(q, kcache, vcache, pack, cap, width, kv, heads, group, scale, start, n, mixed, s);
+}
+
+hipError_t launch_rope_append(const float* qr, const float* kr, const float* vr, uint32_t width, uint32_t kv,
+                              uint32_t head_dim, const float* rcos, const float* rsin, uint32_t start, uint32_t n,
+                              float* q, float* kcache, float* vcache, hipStream_t s) {
+  const uint32_t work = width / 2u + kv;
+  hipLaunchKernelGGL(rope_append_kernel, dim3((work + 255u) / 256u, n), dim3(256), 0, s, qr, kr, vr, width, kv,
+                     head_dim, rcos, rsin, start, q, kcache, vcache);
+  return hipGetLastError();
+}
+
+}  // namespace rh

@@ -1191,11 +1191,12 @@ struct rh_decoder {
   bool fuse_norm = false;    // one-token forwards fold each RMSNorm into the GEMV after it
   bool quant_norm = false;   // batches quantize the normed rows in the norm kernel
   bool quant_ffn = false;    // batches quantize silu(gate) * up in silu_quant_kernel
-  bool quant_attn = false;   // batches quantize the attention output in attention_group_kernel
+  bool quant_attn = false;   // batches give the O matrix the attention output as Q8_K
   bool fuse_output_norm = false;  // one-token forwards fold the output norm into the output matrix's launch
   Q8Dev q8;                  // that activation, for up to `cap` tokens
   float *q = nullptr, *mixed = nullptr, *gate = nullptr, *up = nullptr, *hf = nullptr;
   float* logits = nullptr;
+  float* pack = nullptr;       // a layer's cached rows in the strip attention's operand order
   uint32_t* tokens = nullptr;  // the chunk's token ids
   uint32_t* pick = nullptr;    // argmax: [token, any finite]
   // the output launch's per-workgroup pick partials, and how many the last
@@ -1350,18 +1351,20 @@ rh_status forward_device(rh_decoder* d, const uint32_t* tokens, size_t n, size_t
   const size_t norm_lds = add_norm_lds(w);
   const uint32_t grp = static_cast<uint32_t>(c.head_count / c.head_count_kv);
   const size_t glds = attention_group_lds_floats(grp, start + n) * 4u;
-  const bool grouped = hd == 64u && (grp == 4u || grp == 8u) && glds <= kMaxLdsBytes;
+  const bool groupable = hd == 64u && (grp == 4u || grp == 8u) && glds <= kMaxLdsBytes;
+  const bool strip = attention_strip_ok(hd, start + n, n, groupable), grouped = groupable && !strip;
   // when both producers of the residual delta (the O and down matrices) are
   // k-quant GEMMs over Q8_K operands, they store it token-major and the
   // norms read it coalesced
-  const bool tm = grouped && d->quant_attn && d->quant_ffn && n >= rh_gemm_min_tokens();
+  const bool tm = (strip || grouped) && d->quant_attn && d->quant_ffn && n >= rh_gemm_min_tokens();
   const AddNorm norm_fn = tm ? add_norm_for<false, true>(w) : add_norm_for(w);
   // a batch whose normed rows feed only k-quant GEMMs gets them as Q8_K
   // straight from the norm kernel
   const bool qn = d->quant_norm && n >= 2;
   // with those and the token-major path, the QKV GEMM stores q, k and v
-  // token-major too and the grouped attention does qkv_post_kernel's work
-  const bool rope_in_attn = tm && qn;
+  // token-major too; the grouped attention then does qkv_post_kernel's work,
+  // the strip attention has it done by rope_append_kernel
+  const bool qkv_tm = tm && qn, rope_in_attn = qkv_tm && grouped;
   const AddNorm norm_in = qn ? (tm ? add_norm_for<true, true>(w) : add_norm_for<true>(w)) : norm_fn;
   // the FFN norm that sums a split O launch's planes itself (no combine)
   const AddNorm norm_pl = qn ? add_norm_for<true, true, true>(w) : add_norm_for<false, true, true>(w);
@@ -1372,19 +1375,32 @@ rh_status forward_device(rh_decoder* d, const uint32_t* tokens, size_t n, size_t
                        b.attn_norm, c.rms_norm_eps, 0u, d->normed, d->q8, nullptr, 0u, 0u);
     RHD(hipGetLastError());
     if (qn)
-      RHS(mm_q8(d, n, w, {{b.q, d->qr, n * w}, {b.k, d->kr, n * kv}, {b.v, d->vr, n * kv}}, rope_in_attn));
+      RHS(mm_q8(d, n, w, {{b.q, d->qr, n * w}, {b.k, d->kr, n * kv}, {b.v, d->vr, n * kv}}, qkv_tm));
     else
       RHS(mm(d, d->normed, n, w, {{b.q, d->qr, n * w}, {b.k, d->kr, n * kv}, {b.v, d->vr, n * kv}}));
     float* kc = d->keys + l * c.context_length * kv;
     float* vc = d->values + l * c.context_length * kv;
     SplitOut o_planes;
-    if (!rope_in_attn) {
+    if (qkv_tm && strip) {
+      RHD(launch_rope_append(d->qr, d->kr, d->vr, w, kv, hd, d->rope_cos, d->rope_sin, static_cast<uint32_t>(start), nn,
+                             d->q, kc, vc, s));
+    } else if (!rope_in_attn) {
       const uint32_t work = w / 2u + kv / 2u + kv;
       hipLaunchKernelGGL(qkv_post_kernel, dim3((work + 255u) / 256u, nn), dim3(256), 0, s, d->qr, d->kr, d->vr, nn,
                          w, kv, hd, d->rope_cos, d->rope_sin, static_cast<uint32_t>(start), d->q, kc, vc);
       RHD(hipGetLastError());
     }
-    if (grouped) {
+    if (strip) {
+      RHD(launch_attention_strip(d->q, kc, vc, d->pack, c.context_length, w, kv, hd, scale,
+                                 static_cast<uint32_t>(start), nn, d->mixed, s));
+      if (d->quant_attn) {
+        const Q8Dev q8 = q8_for(d, w);
+        RHD(launch_quantize_super(d->mixed, w, n, q8, s));
+        RHS(mm_q8(d, n, w, {{b.o, d->delta, n * w}}, tm, tm ? &o_planes : nullptr));
+      } else {
+        RHS(mm(d, d->mixed, n, w, {{b.o, d->delta, n * w}}));
+      }
+    } else if (grouped) {
       // the kv head's query heads together; the output as the O matrix's
       // Q8_K operand when it takes one
       const bool qa = d->quant_attn;
@@ -1757,6 +1773,8 @@ rh_status rh_decoder_new(rh_ctx* ctx, const rh_decoder_config* config, const rh_
   ok = ok && dmalloc(&d->keys, cache) == hipSuccess && dmalloc(&d->values, cache) == hipSuccess &&
        dmalloc(&d->logits, c.vocab_size) == hipSuccess && dmalloc(&d->pick, 2) == hipSuccess &&
        dmalloc(&d->pick_parts, c.vocab_size) == hipSuccess &&
+       (!attention_strip_ok(c.head_dim, 2, 2, false) ||
+        dmalloc(&d->pack, attention_pack_floats(c.context_length, d->kv)) == hipSuccess) &&
        dmalloc(&d->count, 2) == hipSuccess;
   if (!ok) {
     rh_decoder_free(d);
@@ -1795,10 +1813,9 @@ rh_status rh_decoder_new(rh_ctx* ctx, const rh_decoder_config* config, const rh_
   for (const rh_decoder::Block& b : d->blocks)
     qffn = qffn && is_kquant_matrix(b.down) && rh_matrix_cols(b.down) == c.feed_forward_length;
   d->quant_ffn = qffn && !(qenv && qenv[0] == '0');
-  // and the attention output, the O matrix's input, where the grouped
-  // attention kernel forms it (head_dim 64, four or eight heads a kv head)
-  const size_t grp = c.head_count_kv ? c.head_count / c.head_count_kv : 0;
-  bool qattn = c.head_dim == 64 && (grp == 4 || grp == 8) && w % 256 == 0;
+  // and the attention output, the O matrix's input, in the grouped attention
+  // kernel or after the strip one
+  bool qattn = w % 256 == 0;
   for (const rh_decoder::Block& b : d->blocks)
     qattn = qattn && is_kquant_matrix(b.o) && rh_matrix_cols(b.o) == w;
   d->quant_attn = qattn && !(qenv && qenv[0] == '0');
@@ -1819,7 +1836,8 @@ void rh_decoder_free(rh_decoder* d) {
   for (void* p : {static_cast<void*>(d->output_norm), static_cast<void*>(d->rope_cos),
                   static_cast<void*>(d->rope_sin), static_cast<void*>(d->keys), static_cast<void*>(d->values),
                   static_cast<void*>(d->logits), static_cast<void*>(d->pick), static_cast<void*>(d->record),
-                  static_cast<void*>(d->count), static_cast<void*>(d->pick_parts)})
+                  static_cast<void*>(d->count), static_cast<void*>(d->pick_parts),
+                  static_cast<void*>(d->pack)})
     if (p) hipFree(p);
   delete d;
 }

@@ -185,6 +185,22 @@ hipError_t launch_gemm(uint32_t type_id, const GemvJobs& jobs, const Q8Dev& q, s
 // `raw` the i32 dots go there instead of the scaled outputs.
 hipError_t launch_gemm_i2s(const GemvJobs& jobs, const Q8Dev& q, size_t tokens, int32_t* raw, hipStream_t s);
 
+// Causal attention of n tokens at positions start.. over the cached rows
+// (attention.hip): q rotated, token-major; the caches hold rows up to
+// start + n; mixed token-major; pack: attention_pack_floats of scratch, whose
+// contents do not outlive the call's work. attention_strip_ok says which
+// batches it takes (rows = start + n; grouped: attention_group_kernel would
+// take the shape).
+bool attention_strip_ok(size_t head_dim, size_t rows, size_t n, bool grouped);
+size_t attention_pack_floats(size_t context, size_t kv);
+hipError_t launch_attention_strip(const float* q, const float* kcache, const float* vcache, float* pack,
+                                  size_t context, uint32_t width, uint32_t kv, uint32_t head_dim, float scale,
+                                  uint32_t start, uint32_t n, float* mixed, hipStream_t s);
+// RoPE of token-major q, k and v from the projections into q and the caches.
+hipError_t launch_rope_append(const float* qr, const float* kr, const float* vr, uint32_t width, uint32_t kv,
+                              uint32_t head_dim, const float* rcos, const float* rsin, uint32_t start, uint32_t n,
+                              float* q, float* kcache, float* vcache, hipStream_t s);
+
 }  // namespace rh
 
 struct rh_ctx;

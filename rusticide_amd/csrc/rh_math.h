@@ -19,7 +19,8 @@
 
 namespace rh {
 
-__host__ __device__ inline float expf_ref(float x) {
+// Entry i of that table.
+__host__ __device__ inline uint64_t exp_table_entry(uint32_t i) {
   constexpr uint64_t kTable[32] = {
     0x3ff0000000000000ULL, 0x3fefd9b0d3158574ULL, 0x3fefb5586cf9890fULL, 0x3fef9301d0125b51ULL,
     0x3fef72b83c7d517bULL, 0x3fef54873168b9aaULL, 0x3fef387a6e756238ULL, 0x3fef1e9df51fdee1ULL,
@@ -30,25 +31,25 @@ __host__ __device__ inline float expf_ref(float x) {
     0x3feee89f995ad3adULL, 0x3feeff76f2fb5e47ULL, 0x3fef199bdd85529cULL, 0x3fef3720dcef9069ULL,
     0x3fef5818dcfba487ULL, 0x3fef7c97337b9b5fULL, 0x3fefa4afa2a490daULL, 0x3fefd0765b6e4540ULL,
   };
+  return kTable[i];
+}
+
+// expf_ref between log(2^-150) and log(2^128), NaN included, with the table
+// entry i given by table(i): a kernel that takes many exponentials keeps the
+// 256 bytes in LDS. No branch keeps its exponentials from overlapping.
+template <typename Table>
+__host__ __device__ inline float expf_ref_inner(float x, Table table) {
   constexpr double kInvLn2N = 0x1.71547652b82fep+0 * 32;
   constexpr double kShift = 0x1.8p+52;
   constexpr double kC0 = 0x1.c6af84b912394p-5 / 32 / 32 / 32;
   constexpr double kC1 = 0x1.ebfce50fac4f3p-3 / 32 / 32;
   constexpr double kC2 = 0x1.62e42ff0c52d6p-1 / 32;
-  const uint32_t bits = __builtin_bit_cast(uint32_t, x);
-  const uint32_t abstop = (bits >> 20) & 0x7ffu;
-  if (abstop >= 0x42bu) {  // |x| >= 88, or x is inf / nan
-    if (bits == 0xff800000u) return 0.0f;
-    if (abstop >= 0x7f8u) return x + x;
-    if (x > 0x1.62e42ep6f) return __builtin_inff();  // past log(2^128)
-    if (x < -0x1.9fe368p6f) return 0.0f;             // below log(2^-150)
-  }
   const double xd = static_cast<double>(x);
   double kd = __builtin_fma(kInvLn2N, xd, kShift);
   const uint64_t ki = __builtin_bit_cast(uint64_t, kd);
   kd -= kShift;
   const double r = __builtin_fma(kInvLn2N, xd, -kd);
-  const uint64_t t = kTable[ki % 32u] + (ki << 47);
+  const uint64_t t = table(static_cast<uint32_t>(ki % 32u)) + (ki << 47);
   const double s = __builtin_bit_cast(double, t);
   const double z = __builtin_fma(kC0, r, kC1);
   const double r2 = r * r;
@@ -56,6 +57,15 @@ __host__ __device__ inline float expf_ref(float x) {
   y = __builtin_fma(z, r2, y);
   y = y * s;
   return static_cast<float>(y);
+}
+
+__host__ __device__ inline float expf_ref(float x) {
+  const float y = expf_ref_inner(x, [](uint32_t i) { return exp_table_entry(i); });
+  if (!(x >= -0x1.9fe368p6f && x <= 0x1.62e42ep6f)) {
+    if (x != x) return x + x;
+    return x > 0.0f ? __builtin_inff() : 0.0f;  // past log(2^128), below log(2^-150)
+  }
+  return y;
 }
 
 }  // namespace rh
