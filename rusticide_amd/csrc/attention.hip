@@ -455,6 +455,265 @@ __global__ __launch_bounds__(kStripThreads, !ONE && HD == 64u ? 4 : 2) void atte
         f32x4{acc[0], acc[1], acc[2], acc[3]};
 }
 
+// One token at position `start` behind more rows than attention_step_lds_kernel
+// holds: two launches, so that neither the key nor the value rows pass through
+// one CU a head. 32 heads of 64 behind 1800 rows: 23 us, against 53 for
+// attention_step_kernel and 30 for one workgroup of 1024 threads a head; 16
+// heads of 128 behind 712: 15.5 us, against 47 for qkv_post_kernel and
+// attention_kernel.
+//
+// step_scores_kernel: a wave takes 16 cached rows of one kv head and forms the
+// scores of up to 16 of its query heads, with the strips' MFMAs. It rotates q
+// and the new key itself (portable/rope.rs:7-23) and appends the new rows to
+// the caches; no wave reads those rows from them. scores: [head][pitch].
+template <uint32_t HD>
+__global__ __launch_bounds__(256) void step_scores_kernel(
+    const float* __restrict__ qr, const float* __restrict__ kr, const float* __restrict__ vr,
+    const float* __restrict__ rcos, const float* __restrict__ rsin, float* kcache, float* vcache, uint32_t kv,
+    uint32_t group, float scale, uint32_t start, uint32_t pitch, float* __restrict__ scores) {
+  constexpr uint32_t MQ = HD / 32u;
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, j = lane & 15u, kq = lane >> 4;
+  const uint32_t r0 = 64u * blockIdx.x + 16u * wave;
+  if (r0 > start) return;
+  const uint32_t kvh = blockIdx.y, jh = 16u * blockIdx.z + j, off = kvh * HD;
+  const uint32_t h = kvh * group + min(jh, group - 1u);
+  const uint32_t row = min(r0 + j, start);
+  const bool fresh = row == start;
+  const float* const kp = (fresh ? kr : kcache + static_cast<size_t>(row) * kv) + off + 8u * kq;
+  const float* const qp = qr + static_cast<size_t>(h) * HD + 8u * kq;
+  const size_t rot = static_cast<size_t>(start) * (HD / 2u) + 4u * kq;
+  f32x4 qf[MQ][2], kf[MQ][2], c[MQ], sn[MQ];
+#pragma unroll
+  for (uint32_t m = 0; m < MQ; m++) {
+    c[m] = *reinterpret_cast<const f32x4*>(rcos + rot + 16u * m);
+    sn[m] = *reinterpret_cast<const f32x4*>(rsin + rot + 16u * m);
+#pragma unroll
+    for (uint32_t u = 0; u < 2u; u++) {
+      qf[m][u] = *reinterpret_cast<const f32x4*>(qp + 32u * m + 4u * u);
+      kf[m][u] = *reinterpret_cast<const f32x4*>(kp + 32u * m + 4u * u);
+    }
+  }
+#pragma unroll
+  for (uint32_t m = 0; m < MQ; m++)
+#pragma unroll
+    for (uint32_t u = 0; u < 2u; u++) {
+      f32x4 y, z;
+#pragma unroll
+      for (uint32_t i = 0; i < 2u; i++) {
+        const float co = c[m][2u * u + i], si = sn[m][2u * u + i];
+        const float ql = qf[m][u][2u * i], qh = qf[m][u][2u * i + 1u];
+        const float kl = kf[m][u][2u * i], kh = kf[m][u][2u * i + 1u];
+        const float qhs = qh * si, qls = ql * si, khs = kh * si, kls = kl * si;
+        y[2u * i] = __builtin_fmaf(ql, co, -qhs);
+        y[2u * i + 1u] = __builtin_fmaf(qh, co, qls);
+        z[2u * i] = __builtin_fmaf(kl, co, -khs);
+        z[2u * i + 1u] = __builtin_fmaf(kh, co, kls);
+      }
+      qf[m][u] = y;
+      if (fresh) kf[m][u] = z;
+    }
+  if (r0 + j == start && blockIdx.z == 0) {
+    float* const kd = kcache + static_cast<size_t>(start) * kv + off + 8u * kq;
+    float* const vd = vcache + static_cast<size_t>(start) * kv + off + 8u * kq;
+#pragma unroll
+    for (uint32_t m = 0; m < MQ; m++)
+#pragma unroll
+      for (uint32_t u = 0; u < 2u; u++) {
+        *reinterpret_cast<f32x4*>(kd + 32u * m + 4u * u) = kf[m][u];
+        *reinterpret_cast<f32x4*>(vd + 32u * m + 4u * u) =
+            *reinterpret_cast<const f32x4*>(vr + off + 8u * kq + 32u * m + 4u * u);
+      }
+  }
+  v4f acc[8];
+#pragma unroll
+  for (uint32_t m = 0; m < MQ; m++)
+#pragma unroll
+    for (uint32_t l = 0; l < 8u; l++)
+      acc[l] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[m][l >> 2][l & 3u], qf[m][l >> 2][l & 3u], m ? acc[l] : v4f{},
+                                                    0, 0, 0);
+  f32x4 sc;
+#pragma unroll
+  for (uint32_t i = 0; i < 4u; i++) {
+    float s = acc[0][i];
+#pragma unroll
+    for (uint32_t l = 1; l < 8u; l++) s += acc[l][i];
+    sc[i] = s;
+  }
+  if constexpr (HD == 64u) sc *= 0.125f;
+  else div_by(sc, scale, 1.0 / static_cast<double>(scale));
+  // rows 4 kq + i of the wave's 16 for query head j (the pitch has room for
+  // the rows past the last)
+  if (jh < group) *reinterpret_cast<f32x4*>(scores + static_cast<size_t>(h) * pitch + r0 + 4u * kq) = sc;
+}
+
+// step_mix_kernel: a workgroup takes kStepD output lanes of one query head:
+// the softmax over the head's scores (every such workgroup forms the same
+// one), with its slice of the value rows on its way into LDS meanwhile; then
+// the lanes' chains of fused adds over the rows, on one wave.
+// What bounds it: that chain. A dependent fused add takes 4.2 cycles, a lane's
+// LDS reads of four rows' values and weights about as long again each: 12
+// cycles a row, 10.3 us of 15.3 behind 1800 rows, the ordered sum 1.1.
+constexpr uint32_t kStepD = 8;
+constexpr uint32_t kMixThreads = 512;
+constexpr uint32_t kMixEarly = 2;  // pieces of value rows a thread loads before the softmax
+
+// LDS: the value slice, four rows x kStepD lanes a block of 32 floats, the
+// weights, a reduction.
+constexpr size_t step_mix_lds_bytes(size_t rows) {
+  return 4u * (((rows + 3u) / 4u) * 32u + wave_sum_floats(static_cast<uint32_t>(rows)) + 16u);
+}
+
+// Slot of output lane d in block r4: exchanged so that the stores of a wave
+// (a lane's four rows of four lanes, transposed) fall on distinct banks.
+__device__ __forceinline__ uint32_t mix_slot(uint32_t r4, uint32_t d) { return 8u * r4 + (d ^ ((r4 >> 1) & 3u)); }
+
+template <uint32_t HD>
+__global__ __launch_bounds__(kMixThreads) void step_mix_kernel(const float* __restrict__ scores,
+                                                               const float* __restrict__ vcache, uint32_t kv,
+                                                               uint32_t group, uint32_t rows, uint32_t pitch,
+                                                               float* __restrict__ mixed) {
+  constexpr uint32_t SL = HD / kStepD, NWV = kMixThreads / 64u;
+  extern __shared__ __align__(16) float sh[];
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+  const uint32_t r4s = (rows + 3u) / 4u;
+  f32x4* const vt = reinterpret_cast<f32x4*>(sh);              // [r4s][8] (mix_slot)
+  float* const ws = sh + r4s * 32u;                     // exps, then weights (wave_sum_index)
+  float* const red = ws + wave_sum_floats(rows);         // [8] maxima, [8] the sum
+  // workgroups go to the eight XCDs in turn: the slices of a head, which share
+  // the lines of its values, on one of them
+  const uint32_t H = gridDim.x / SL, b = blockIdx.x;
+  const uint32_t h = H % 8u == 0 ? (b & 7u) + 8u * ((b >> 3) / SL) : b / SL;
+  const uint32_t slice = H % 8u == 0 ? (b >> 3) % SL : b % SL, off = (h / group) * HD + kStepD * slice;
+  const float* const sp = scores + static_cast<size_t>(h) * pitch;
+
+  // four rows x four lanes of values a piece: piece f is block f / 2, lanes 4 (f % 2) ..
+  const uint32_t pieces = 2u * r4s;
+  auto load_piece = [&](f32x4 (&x)[4], uint32_t f) {
+    const uint32_t r = 4u * (f >> 1), o = off + 4u * (f & 1u);
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; k++)
+      x[k] = *reinterpret_cast<const f32x4*>(vcache + static_cast<size_t>(min(r + k, rows - 1u)) * kv + o);
+  };
+  auto store_piece = [&](const f32x4 (&x)[4], uint32_t f) {
+    if (f >= pieces) return;
+#pragma unroll
+    for (uint32_t u = 0; u < 4u; u++)
+      vt[mix_slot(f >> 1, 4u * (f & 1u) + u)] = f32x4{x[0][u], x[1][u], x[2][u], x[3][u]};
+  };
+  // a thread's first four scores, then its first values: loads return in order
+  f32x4 s0 = *reinterpret_cast<const f32x4*>(sp + min(4u * tid, 4u * (r4s - 1u)));
+  f32x4 early[kMixEarly][4];
+#pragma unroll
+  for (uint32_t k = 0; k < kMixEarly; k++) load_piece(early[k], tid + k * kMixThreads);
+
+  // ---- softmax (norm.rs:17-30)
+  float mx = -INFINITY;
+  for (uint32_t i = 4u * tid; i < rows; i += 4u * kMixThreads) {
+    const f32x4 x = i == 4u * tid ? s0 : *reinterpret_cast<const f32x4*>(sp + i);
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; k++)
+      if (i + k < rows) mx = fmaxf(mx, x[k]);
+  }
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+  if (lane == 0) red[wave] = mx;
+  __syncthreads();
+  mx = red[0];
+#pragma unroll
+  for (uint32_t k = 1; k < NWV; k++) mx = fmaxf(mx, red[k]);
+  // the exps; the sum's identity up to the end of the last chunk of 32
+  for (uint32_t i = 4u * tid; i < ((rows + 31u) & ~31u); i += 4u * kMixThreads) {
+    f32x4 x = s0;
+    if (i != 4u * tid) x = *reinterpret_cast<const f32x4*>(sp + min(i, 4u * (r4s - 1u)));
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; k++) {
+      const float e = expf_ref(x[k] - mx);
+      x[k] = i + k < rows ? e : -0.0f;
+    }
+    *reinterpret_cast<f32x4*>(ws + wave_sum_index(i)) = x;
+  }
+#pragma unroll
+  for (uint32_t k = 0; k < kMixEarly; k++) store_piece(early[k], tid + k * kMixThreads);
+  __syncthreads();
+  if (wave == 0) {
+    const float sum = ordered_sum_wave(ws, rows, 0.0f);
+    if (lane == 0) red[8] = sum;
+  } else {
+    for (uint32_t f = kMixEarly * kMixThreads + tid - 64u; f < pieces; f += kMixThreads - 64u) {
+      f32x4 x[4];
+      load_piece(x, f);
+      store_piece(x, f);
+    }
+  }
+  __syncthreads();
+  {
+    const float sum = red[8];
+    const double inv = 1.0 / static_cast<double>(sum);
+    for (uint32_t i = 4u * tid; i < rows; i += 4u * kMixThreads) {
+      f32x4* const w = reinterpret_cast<f32x4*>(ws + wave_sum_index(i));
+      f32x4 x = *w;
+      div_by(x, sum, inv);
+      *w = x;
+    }
+  }
+  __syncthreads();
+  if (wave != 0) return;
+
+  // ---- value mix (float.rs:52-62): eight blocks of four rows in flight (LDS
+  // reads are counted up to 15), each read again as soon as it is added, 32
+  // rows on; a lane's reads sit at fixed offsets of four addresses (one for
+  // each exchange of mix_slot)
+  if (lane >= kStepD) return;
+  float acc = 0.0f;
+  uint32_t vo[4];
+#pragma unroll
+  for (uint32_t i = 0; i < 4u; i++) vo[i] = lane ^ i;
+  const f32x4* const wt = reinterpret_cast<const f32x4*>(ws);
+  f32x4 v[8], w[8];
+  auto add = [&](uint32_t i) {
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; k++) acc = __builtin_fmaf(v[i][k], w[i][k], acc);
+  };
+  const uint32_t chunks = rows >> 5;
+  if (chunks) {
+#pragma unroll
+    for (uint32_t i = 0; i < 8u; i++) {
+      v[i] = vt[vo[i >> 1] + 8u * i];
+      w[i] = wt[i];
+    }
+    for (uint32_t c = 1; c < chunks; c++) {
+#pragma unroll
+      for (uint32_t i = 0; i < 4u; i++) vo[i] += 64u;
+#pragma unroll
+      for (uint32_t i = 0; i < 8u; i++) {
+        add(i);
+        v[i] = vt[vo[i >> 1] + 8u * i];
+        w[i] = wt[9u * c + i];
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < 8u; i++) add(i);
+  }
+  for (uint32_t r = 32u * chunks; r < rows; r++)
+    acc = __builtin_fmaf(reinterpret_cast<const float*>(vt + mix_slot(r >> 2, lane))[r & 3u], ws[wave_sum_index(r)],
+                         acc);
+  mixed[static_cast<size_t>(h) * HD + kStepD * slice + lane] = acc;
+}
+
+template <uint32_t HD>
+hipError_t launch_step(const float* qr, const float* kr, const float* vr, const float* rcos, const float* rsin,
+                       float* kcache, float* vcache, uint32_t heads, uint32_t kv, uint32_t group, float scale,
+                       uint32_t start, float* scores, uint32_t pitch, float* mixed, hipStream_t s) {
+  hipLaunchKernelGGL((step_scores_kernel<HD>), dim3(start / 64u + 1u, kv / HD, (group + 15u) / 16u), dim3(256), 0, s,
+                     qr, kr, vr, rcos, rsin, kcache, vcache, kv, group, scale, start, pitch, scores);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((step_mix_kernel<HD>), dim3(heads * (HD / kStepD)), dim3(kMixThreads),
+                     step_mix_lds_bytes(start + 1u), s, scores, vcache, kv, group, start + 1u, pitch, mixed);
+  return hipGetLastError();
+}
+
 // q/k/v from the projections, token-major: q and k rotated
 // (portable/rope.rs:7-23), k and v into the cache at positions start + t. One
 // thread per rotation pair (q, k) or pair of value elements.
@@ -552,6 +811,24 @@ hipError_t launch_attention_strip(const float* q, const float* kcache, const flo
   if (head_dim == 64u)
     return launch_strips<64>(q, kcache, vcache, pack, cap, width, kv, heads, group, scale, start, n, mixed, s);
   return launch_strips<128>(q, kcache, vcache, pack, cap, width, kv, heads, group, scale, start, n, mixed, s);
+}
+
+bool attention_step_long_ok(size_t head_dim, size_t rows) {
+  return (head_dim == 64u || head_dim == 128u) && rows <= 65536u && step_mix_lds_bytes(rows) <= kLdsBytes;
+}
+
+size_t attention_step_pitch(size_t context) { return (context + 63u) & ~size_t{63}; }
+
+hipError_t launch_attention_step_long(const float* qr, const float* kr, const float* vr, const float* rcos,
+                                      const float* rsin, float* kcache, float* vcache, uint32_t heads, uint32_t kv,
+                                      uint32_t head_dim, float scale, uint32_t start, float* scores, uint32_t pitch,
+                                      float* mixed, hipStream_t s) {
+  const uint32_t group = heads / (kv / head_dim);
+  if (head_dim == 64u)
+    return launch_step<64>(qr, kr, vr, rcos, rsin, kcache, vcache, heads, kv, group, scale, start, scores, pitch,
+                           mixed, s);
+  return launch_step<128>(qr, kr, vr, rcos, rsin, kcache, vcache, heads, kv, group, scale, start, scores, pitch, mixed,
+                          s);
 }
 
 hipError_t launch_rope_append(const float* qr, const float* kr, const float* vr, uint32_t width, uint32_t kv,

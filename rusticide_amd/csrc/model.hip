@@ -1197,6 +1197,7 @@ struct rh_decoder {
   float *q = nullptr, *mixed = nullptr, *gate = nullptr, *up = nullptr, *hf = nullptr;
   float* logits = nullptr;
   float* pack = nullptr;       // a layer's cached rows in the strip attention's operand order
+  float* scores = nullptr;     // one token's attention scores, [head][attention_step_pitch]
   uint32_t* tokens = nullptr;  // the chunk's token ids
   uint32_t* pick = nullptr;    // argmax: [token, any finite]
   // the output launch's per-workgroup pick partials, and how many the last
@@ -1520,6 +1521,11 @@ rh_status forward_one_fused(rh_decoder* d, const uint32_t* tokens, size_t start,
       void* args[] = {&qr, &kr, &vr, &rc, &rs, &kc, &vc, &kv32, &gr, &sc, &st, &mixed};
       RHD(hipLaunchKernel(k, dim3(static_cast<uint32_t>(c.head_count)), dim3(kAttnThreads), args,
                           attention_step_lds_bytes(nk), s));
+    } else if (attention_step_long_ok(hd, start + 1u) && tuning().attn_lds) {
+      RHD(launch_attention_step_long(d->qr, d->kr, d->vr, d->rope_cos, d->rope_sin, kc, vc,
+                                     static_cast<uint32_t>(c.head_count), kv, hd, scale, static_cast<uint32_t>(start),
+                                     d->scores, static_cast<uint32_t>(attention_step_pitch(c.context_length)),
+                                     d->mixed, s));
     } else if (hd == 64u) {
       hipLaunchKernelGGL(attention_step_kernel, dim3(static_cast<uint32_t>(c.head_count)), dim3(kAttnThreads),
                          att_lds, s, d->qr, d->kr, d->vr, d->rope_cos, d->rope_sin, kc, vc, kv, group, scale,
@@ -1775,6 +1781,7 @@ rh_status rh_decoder_new(rh_ctx* ctx, const rh_decoder_config* config, const rh_
        dmalloc(&d->pick_parts, c.vocab_size) == hipSuccess &&
        (!attention_strip_ok(c.head_dim, 2, 2, false) ||
         dmalloc(&d->pack, attention_pack_floats(c.context_length, d->kv)) == hipSuccess) &&
+       dmalloc(&d->scores, c.head_count * attention_step_pitch(c.context_length)) == hipSuccess &&
        dmalloc(&d->count, 2) == hipSuccess;
   if (!ok) {
     rh_decoder_free(d);
@@ -1836,7 +1843,7 @@ void rh_decoder_free(rh_decoder* d) {
   for (void* p : {static_cast<void*>(d->output_norm), static_cast<void*>(d->rope_cos),
                   static_cast<void*>(d->rope_sin), static_cast<void*>(d->keys), static_cast<void*>(d->values),
                   static_cast<void*>(d->logits), static_cast<void*>(d->pick), static_cast<void*>(d->record),
-                  static_cast<void*>(d->count), static_cast<void*>(d->pick_parts),
+                  static_cast<void*>(d->count), static_cast<void*>(d->pick_parts), static_cast<void*>(d->scores),
                   static_cast<void*>(d->pack)})
     if (p) hipFree(p);
   delete d;

@@ -196,6 +196,15 @@ size_t attention_pack_floats(size_t context, size_t kv);
 hipError_t launch_attention_strip(const float* q, const float* kcache, const float* vcache, float* pack,
                                   size_t context, uint32_t width, uint32_t kv, uint32_t head_dim, float scale,
                                   uint32_t start, uint32_t n, float* mixed, hipStream_t s);
+// One token's RoPE, KV append and attention over start + 1 rows, from the raw
+// projections; attention_step_long_ok says which rows it takes. scores holds
+// heads rows of `pitch` floats (attention_step_pitch of the context).
+bool attention_step_long_ok(size_t head_dim, size_t rows);
+size_t attention_step_pitch(size_t context);
+hipError_t launch_attention_step_long(const float* qr, const float* kr, const float* vr, const float* rcos,
+                                      const float* rsin, float* kcache, float* vcache, uint32_t heads, uint32_t kv,
+                                      uint32_t head_dim, float scale, uint32_t start, float* scores, uint32_t pitch,
+                                      float* mixed, hipStream_t s);
 // RoPE of token-major q, k and v from the projections into q and the caches.
 hipError_t launch_rope_append(const float* qr, const float* kr, const float* vr, uint32_t width, uint32_t kv,
                               uint32_t head_dim, const float* rcos, const float* rsin, uint32_t start, uint32_t n,

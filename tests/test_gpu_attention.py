@@ -57,3 +57,10 @@ def test_prompt_chunks(ctx, heads, kv_heads, head_dim):
 @pytest.mark.parametrize("heads,kv_heads,head_dim", [(8, 1, 64), (4, 1, 128)])
 def test_long_prompt(ctx, heads, kv_heads, head_dim):
     check(ctx, config(heads, kv_heads, head_dim, 2600), [2400, 90, 37, 40], 5)
+
+
+# single tokens behind a prompt, at and around whole tiles of 128 and 256 rows
+@pytest.mark.parametrize("heads,kv_heads,head_dim", [(8, 1, 64), (12, 4, 64), (4, 1, 128), (8, 8, 128)])
+@pytest.mark.parametrize("prompt", [126, 222, 254, 510, 1000])
+def test_steps_behind_a_prompt(ctx, heads, kv_heads, head_dim, prompt):
+    check(ctx, config(heads, kv_heads, head_dim, 1100), [prompt, 1, 1, 1, 1], prompt)
