@@ -1196,6 +1196,8 @@ struct rh_decoder {
   Q8Dev q8;                  // that activation, for up to `cap` tokens
   float *q = nullptr, *mixed = nullptr, *gate = nullptr, *up = nullptr, *hf = nullptr;
   float* logits = nullptr;
+  float* host_logits = nullptr;    // page-locked: a forward's logits on their way to the caller
+  uint32_t* host_token = nullptr;  // page-locked: a one-token forward's id
   float* pack = nullptr;       // a layer's cached rows in the strip attention's operand order
   float* scores = nullptr;     // one token's attention scores, [head][attention_step_pitch]
   uint32_t* tokens = nullptr;  // the chunk's token ids
@@ -1583,6 +1585,19 @@ rh_status forward_one_fused(rh_decoder* d, const uint32_t* tokens, size_t start,
   return RH_OK;
 }
 
+// logits[0..m) to page-locked host memory. A copy command to the caller's
+// pageable memory goes through the runtime's staging with a wait of its own;
+// this one is a launch like the ones before it (rh_decoder_forward_batch).
+__global__ __launch_bounds__(256) void logits_out_kernel(const float* __restrict__ logits, uint32_t m,
+                                                         float* __restrict__ out) {
+  const uint32_t i = 4u * (blockIdx.x * 256u + threadIdx.x);
+  if (i + 4u <= m) {
+    *reinterpret_cast<f32x4*>(out + i) = *reinterpret_cast<const f32x4*>(logits + i);
+    return;
+  }
+  for (uint32_t e = i; e < m; e++) out[e] = logits[e];
+}
+
 }  // namespace
 
 extern "C" {
@@ -1779,6 +1794,8 @@ rh_status rh_decoder_new(rh_ctx* ctx, const rh_decoder_config* config, const rh_
   ok = ok && dmalloc(&d->keys, cache) == hipSuccess && dmalloc(&d->values, cache) == hipSuccess &&
        dmalloc(&d->logits, c.vocab_size) == hipSuccess && dmalloc(&d->pick, 2) == hipSuccess &&
        dmalloc(&d->pick_parts, c.vocab_size) == hipSuccess &&
+       hipHostMalloc(reinterpret_cast<void**>(&d->host_logits), c.vocab_size * 4, hipHostMallocDefault) == hipSuccess &&
+       hipHostMalloc(reinterpret_cast<void**>(&d->host_token), 64, hipHostMallocDefault) == hipSuccess &&
        (!attention_strip_ok(c.head_dim, 2, 2, false) ||
         dmalloc(&d->pack, attention_pack_floats(c.context_length, d->kv)) == hipSuccess) &&
        dmalloc(&d->scores, c.head_count * attention_step_pitch(c.context_length)) == hipSuccess &&
@@ -1846,6 +1863,8 @@ void rh_decoder_free(rh_decoder* d) {
                   static_cast<void*>(d->count), static_cast<void*>(d->pick_parts), static_cast<void*>(d->scores),
                   static_cast<void*>(d->pack)})
     if (p) hipFree(p);
+  if (d->host_logits) hipHostFree(d->host_logits);
+  if (d->host_token) hipHostFree(d->host_token);
   delete d;
 }
 
@@ -1929,11 +1948,26 @@ rh_status rh_decoder_forward_batch(rh_decoder* d, const uint32_t* tokens, size_t
   if (start != d->cached) return RH_ERR_CACHE_POSITION;  // cache.rs:56-61
   if (hipSetDevice(ctx_device(d->ctx)) != hipSuccess) return RH_ERR_DEVICE;
   if (ensure_acts(d, n) != hipSuccess) return RH_ERR_OUT_OF_MEMORY;
-  RHD(hipMemcpyAsync(d->tokens, tokens, n * 4, hipMemcpyHostToDevice, d->stream));
-  RHS(forward_cached(d, n, start));
+  // one token's id is read from page-locked memory by the embedding itself,
+  // and the logits come back through it (every call waits for its own work,
+  // so the buffer is free again): 44 us a call less of wall clock than with
+  // two copy commands (1777 tokens and 40 steps through two layers of 32
+  // heads of 64: 7264 us against 9037)
+  if (n == 1) {
+    *d->host_token = tokens[0];
+    RHS(forward_device(d, d->host_token, n, start));
+  } else {
+    RHD(hipMemcpyAsync(d->tokens, tokens, n * 4, hipMemcpyHostToDevice, d->stream));
+    RHS(forward_cached(d, n, start));
+  }
   const size_t m = logits_len < d->c.vocab_size ? logits_len : d->c.vocab_size;
-  if (m) RHD(hipMemcpyAsync(logits, d->logits, m * 4, hipMemcpyDeviceToHost, d->stream));
+  if (m) {
+    hipLaunchKernelGGL(logits_out_kernel, dim3(static_cast<uint32_t>((m + 1023u) / 1024u)), dim3(256), 0, d->stream,
+                       d->logits, static_cast<uint32_t>(m), d->host_logits);
+    RHD(hipGetLastError());
+  }
   RHD(hipStreamSynchronize(d->stream));
+  if (m) std::memcpy(logits, d->host_logits, m * 4);
   return RH_OK;
 }
 
