@@ -246,7 +246,7 @@ __device__ __forceinline__ void split_fixup(const GemvJobs& jobs, const SplitTer
 // Planes: Q4_K's w = sc*q is split along the scale, sc = 8*sh + sl (sh, sl
 // in 0..7), so each plane byte sh*q or sl*q (at most 105) is one packed
 // 16-bit multiply of four nibbles; isum = 8*hi + lo. Q6_K keeps w = sc*(q-32)
-// = 128*hi + lo. Both sums are exact in i32.
+// = 256*hi + lo. Both sums are exact in i32.
 //
 // The matrices are in the unit layout (rh_device.h): the lane's pieces of a
 // block sit at fixed 16-byte-aligned offsets of its group of 16 blocks.
@@ -316,24 +316,25 @@ __device__ __forceinline__ void lane_planes(const LaneRaw<12>& x, uint32_t kk, u
   }
 }
 
-// Q6_K: four 6-bit bytes q as w = sc * (q - 32) in hi/lo planes (w = 128*hi
-// + lo, lo in 0..127). The bytes are spread into 16-bit lanes and multiplied
-// with one packed multiply-add each ((q - 32)*sc fits i16: |w| <= 4096),
-// then the planes' bytes are gathered back with v_perm_b32.
+// Q6_K: four 6-bit bytes q as w = sc * (q - 32) in hi/lo planes (w = 256*hi
+// + lo, lo in -128..127). The bytes are spread into 16-bit lanes and multiplied
+// with one packed multiply-add each, which gives w + 128 (|w| <= 4096): its
+// high byte is hi, its low byte less 128 lo, gathered with v_perm_b32. Seven
+// operations where a split at 128 took nine (2048 x 5632 for 509 tokens, bound
+// by this decoding: 50.0 against 52.8 us).
 __device__ __forceinline__ void q6_split(uint32_t q, int32_t sc, uint32_t& hi, uint32_t& lo) {
   typedef int16_t i16x2 __attribute__((ext_vector_type(2)));
   const i16x2 scv{static_cast<int16_t>(sc), static_cast<int16_t>(sc)};
-  const i16x2 off{static_cast<int16_t>(-32 * sc), static_cast<int16_t>(-32 * sc)};
+  const i16x2 off{static_cast<int16_t>(128 - 32 * sc), static_cast<int16_t>(128 - 32 * sc)};
   // bytes 0,2 -> lanes of qe; bytes 1,3 -> lanes of qo (zero high bytes)
   const uint32_t qe = __builtin_amdgcn_perm(0u, q, 0x0c020c00u);
   const uint32_t qo = __builtin_amdgcn_perm(0u, q, 0x0c030c01u);
   const i16x2 we = __builtin_bit_cast(i16x2, qe) * scv + off;
   const i16x2 wo = __builtin_bit_cast(i16x2, qo) * scv + off;
   const uint32_t ue = __builtin_bit_cast(uint32_t, we), uo = __builtin_bit_cast(uint32_t, wo);
-  // bytes (we.lo, wo.lo, we.hi, wo.hi) -> low byte of each 16-bit product
-  lo = __builtin_amdgcn_perm(uo, ue, 0x06020400u) & 0x7F7F7F7Fu;
-  const i16x2 he = we >> static_cast<int16_t>(7), ho = wo >> static_cast<int16_t>(7);
-  hi = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, ho), __builtin_bit_cast(uint32_t, he), 0x06020400u);
+  // the low, then the high byte of each: (we.0, wo.0, we.1, wo.1)
+  lo = __builtin_amdgcn_perm(uo, ue, 0x06020400u) ^ 0x80808080u;
+  hi = __builtin_amdgcn_perm(uo, ue, 0x07030501u);
 }
 
 __device__ __forceinline__ void lane_planes(const LaneRaw<14>& x, uint32_t kk, uint32_t g, v4i& hi, v4i& lo) {
@@ -515,7 +516,7 @@ __global__ __launch_bounds__(256) void gemm_kq_rows_kernel(GemvJobs jobs, Q8Dev 
       for (int i = 0; i < 16; i++) {
         const uint32_t m = 8u * static_cast<uint32_t>(i >> 2) + 4u * g + static_cast<uint32_t>(i & 3);
         const float2 dd = rowdT[wave * 32u + m];
-        const int32_t isum = FMT == 12 ? (acc_h[t][i] << 3) + acc_l[t][i] : (acc_h[t][i] << 7) + acc_l[t][i];
+        const int32_t isum = FMT == 12 ? (acc_h[t][i] << 3) + acc_l[t][i] : (acc_h[t][i] << 8) + acc_l[t][i];
         float term;
         if constexpr (FMT == 12) {
           // int_dot.rs:169: d8 * d.mul_add(isum, -(dmin * msum))
