@@ -457,7 +457,7 @@ __global__ __launch_bounds__(kStripThreads, !ONE && HD == 64u ? 4 : 2) void atte
 
 // One token at position `start` behind more rows than attention_step_lds_kernel
 // holds: two launches, so that neither the key nor the value rows pass through
-// one CU a head. 32 heads of 64 behind 1800 rows: 23 us, against 53 for
+// one CU a head. 32 heads of 64 behind 1800 rows: 23-25 us, against 53 for
 // attention_step_kernel and 30 for one workgroup of 1024 threads a head; 16
 // heads of 128 behind 712: 15.5 us, against 47 for qkv_post_kernel and
 // attention_kernel.
