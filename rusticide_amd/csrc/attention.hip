@@ -213,6 +213,23 @@ __global__ __launch_bounds__(256) void pack_kv_kernel(const float* __restrict__ 
   }
 }
 
+// Workgroup b's tile of tokens and run of heads, for `tiles` tiles of hx runs.
+// Workgroups go to the eight XCDs in turn: from eight tiles on, a tile's heads
+// stay on one XCD; with fewer, no XCD is without work (8 tokens behind 2350
+// rows, 40 heads of 64 over 8 kv heads, one tile: 41 us a layer less than with
+// its 40 workgroups on one XCD's 32 CUs).
+struct StripPlace {
+  uint32_t tile, heads;
+};
+__host__ __device__ constexpr uint32_t strip_turn(uint32_t tiles) { return tiles < 8u ? tiles : 8u; }
+__host__ __device__ constexpr uint32_t strip_grid(uint32_t tiles, uint32_t hx) {
+  return hx * ((tiles + strip_turn(tiles) - 1u) / strip_turn(tiles) * strip_turn(tiles));
+}
+__host__ __device__ constexpr StripPlace strip_place(uint32_t b, uint32_t tiles, uint32_t hx) {
+  const uint32_t turn = strip_turn(tiles), k = b / turn;
+  return {b % turn + turn * (k / hx), k % hx};
+}
+
 // A workgroup owns 16 query rows -- 16 >> hs_log tokens of (1 << hs_log)
 // heads that share a kv head -- over all their cached rows, three phases
 // apart by a barrier:
@@ -252,11 +269,10 @@ __global__ __launch_bounds__(kStripThreads, !ONE && HD == 64u ? 4 : 2) void atte
   const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(tid >> 6)));
   const uint32_t j = lane & 15u, kq = lane >> 4;        // the lane's query row (or operand row) and k
   const uint32_t tps = kStripQ >> hs_log;               // tokens a strip
-  // the longest strips first
-  const uint32_t hx = heads >> hs_log, ty = (blockIdx.x & 7u) + 8u * ((blockIdx.x >> 3) / hx);
-  if (ty >= tiles) return;
-  const uint32_t t0 = (tile0 + tiles - 1u - ty) * tps;
-  const uint32_t h0 = ((blockIdx.x >> 3) % hx) << hs_log, off = (h0 / group) * HD;
+  const StripPlace place = strip_place(blockIdx.x, tiles, heads >> hs_log);
+  if (place.tile >= tiles) return;
+  const uint32_t t0 = (tile0 + tiles - 1u - place.tile) * tps;  // the longest strips first
+  const uint32_t h0 = place.heads << hs_log, off = (h0 / group) * HD;
   const uint32_t tj = t0 + (j >> hs_log), hj = h0 + (j & ((1u << hs_log) - 1u));
   const uint32_t tc = min(tj, n - 1u);                  // past the batch: its last token, not stored
   const uint32_t pos = start + tc;                      // the last cached row of query row j
@@ -774,7 +790,7 @@ hipError_t launch_strips(const float* q, const float* kcache, const float* vcach
     if (t0 == t1) continue;
     const uint32_t groups = (start + std::min(t1 * tps, n) - 1u) / 16u + 1u;
     const auto fn = groups > kStripHalfGroups ? attention_strip_kernel<HD, true> : attention_strip_kernel<HD, false>;
-    hipLaunchKernelGGL(fn, dim3((heads >> hs_log) * ((t1 - t0 + 7u) & ~7u)), dim3(kStripThreads),
+    hipLaunchKernelGGL(fn, dim3(strip_grid(t1 - t0, heads >> hs_log)), dim3(kStripThreads),
                        strip_lds_bytes(groups), s, q, pack, vpack, vcache, cap, width, kv, heads, hs_log, group, scale,
                        start, n, t0, t1 - t0, strip_stride(groups), mixed);
     const hipError_t e = hipGetLastError();
@@ -841,3 +857,15 @@ hipError_t launch_rope_append(const float* qr, const float* kr, const float* vr,
 }
 
 }  // namespace rh
+
+extern "C" {
+
+// Test hook: workgroup b's tile and run of heads; returns the grid.
+uint32_t rh_strip_place_host(uint32_t b, uint32_t tiles, uint32_t hx, uint32_t* tile, uint32_t* heads) {
+  const rh::StripPlace at = rh::strip_place(b, tiles, hx);
+  *tile = at.tile;
+  *heads = at.heads;
+  return rh::strip_grid(tiles, hx);
+}
+
+}  // extern "C"
