@@ -214,19 +214,23 @@ __global__ __launch_bounds__(256) void pack_kv_kernel(const float* __restrict__ 
 }
 
 // Workgroup b's tile of tokens and run of heads, for `tiles` tiles of hx runs.
-// Workgroups go to the eight XCDs in turn: from eight tiles on, a tile's heads
-// stay on one XCD; with fewer, no XCD is without work (8 tokens behind 2350
-// rows, 40 heads of 64 over 8 kv heads, one tile: 41 us a layer less than with
-// its 40 workgroups on one XCD's 32 CUs).
+// Workgroups go to the eight XCDs in turn: a tile's heads stay on one XCD while
+// its 32 CUs hold them or every XCD has a tile; otherwise they go round (8
+// tokens behind 2350 rows, 40 heads of 64 over 8 kv heads, one tile: 41 us a
+// layer less; 32 heads over 32, 9 tokens: 4 less behind 2000 rows, 1 more at 9;
+// 16 heads of 128, one tile: 1 more at 9, 0 at 700).
 struct StripPlace {
   uint32_t tile, heads;
 };
-__host__ __device__ constexpr uint32_t strip_turn(uint32_t tiles) { return tiles < 8u ? tiles : 8u; }
+__host__ __device__ constexpr uint32_t strip_turn(uint32_t tiles, uint32_t hx) {
+  return tiles < 8u && hx >= 32u ? tiles : 8u;
+}
 __host__ __device__ constexpr uint32_t strip_grid(uint32_t tiles, uint32_t hx) {
-  return hx * ((tiles + strip_turn(tiles) - 1u) / strip_turn(tiles) * strip_turn(tiles));
+  const uint32_t turn = strip_turn(tiles, hx);
+  return hx * ((tiles + turn - 1u) / turn * turn);
 }
 __host__ __device__ constexpr StripPlace strip_place(uint32_t b, uint32_t tiles, uint32_t hx) {
-  const uint32_t turn = strip_turn(tiles), k = b / turn;
+  const uint32_t turn = strip_turn(tiles, hx), k = b / turn;
   return {b % turn + turn * (k / hx), k % hx};
 }
 
