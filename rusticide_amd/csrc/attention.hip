@@ -805,18 +805,43 @@ hipError_t launch_strips(const float* q, const float* kcache, const float* vcach
 
 }  // namespace
 
-// Rows from which strips are the faster where attention_group_kernel takes the
-// shape: it needs no packing, no RoPE and no quantize launch. Two layers of a
-// 64-token batch, wall clock, 32/4 heads of 64: 219 us against 222 at 192 rows,
-// 219 against 227 at 256, 227 against 261 at 512; 16 tokens: 203 against 200
-// at 208 rows, 205 against 211 at 272. Heads of 128 (attention_kernel) gain at
-// every length: 224 against 233 us at 64 rows.
-constexpr size_t kStripMinRows = 224;
-
-bool attention_strip_ok(size_t head_dim, size_t rows, size_t n, bool grouped) {
-  return (head_dim == 64u || head_dim == 128u) && rows <= 16u * kStripMaxGroups && n >= 2u &&
-         (!grouped || rows >= kStripMinRows);
+// Rows (cached and new) from which a batch of n tokens takes strips: the
+// lines where they and the kernels they replace measured the same. Strips cost
+// a packing launch more, and where the O matrix's operand is `quantized` its
+// launch; the others cost a workgroup per token and head (attention_kernel) or
+// kv head (attention_group_kernel, `grouped`), free until they fill the chip.
+// us a layer, strips less the other kernels, 32 heads of 64 unless stated:
+//   grouped: eight heads a kv head -3 from 224 rows on (8 tokens); four, up to
+//   8 tokens and quantized, +2 at 224 and -3 at 800, 12 tokens +2 at 260 and
+//   -2 at 350, 48 tokens -3 at 224. 64 tokens, eight heads: 219 against 222 us
+//   at 192 rows for two layers, which is why nothing here lies below 224.
+//   token_major (k-quant GEMMs store q, k, v and the O rows token-major for
+//   strips, row-major for attention_kernel): -1 to -6 from the first row on.
+//   others, up to 256 (token, head) pairs, where the packing's share grows
+//   with the kv width: 2 kv heads +1 at 700 rows, -1 at 1000; 16 kv heads +2 at
+//   1000, -1 at 1400; 32 kv heads +3 at 1200, 0 at 1700. 384 pairs: +1 to +3 at
+//   400, -4 at 1000; 768: +1 at 120, -2 at 260; 1536: -3 at 48.
+//   16 heads of 128: 8 tokens +4 at 8 rows, +1 at 120, -3 at 224; 32 tokens +2
+//   at 32, -9 at 180; 48 tokens -3 at 48.
+size_t attention_strip_rows(size_t head_dim, size_t heads, size_t kv_heads, size_t n, bool grouped, bool quantized,
+                            bool token_major) {
+  const size_t pairs = n * heads;
+  if (grouped) {
+    if (heads / kv_heads == 8u || n >= 24u) return 224u;
+    return quantized && n <= 8u ? 640u : 320u;
+  }
+  if (token_major) return 0u;
+  if (head_dim == 128u) return pairs <= 256u ? 144u : pairs < 768u ? 64u : 0u;
+  return pairs <= 256u ? 768u + kv_heads * head_dim / 2u : pairs <= 512u ? 512u : pairs < 1536u ? 160u : 0u;
 }
+
+bool attention_strip_ok(size_t head_dim, size_t heads, size_t kv_heads, size_t rows, size_t n, bool grouped,
+                        bool quantized, bool token_major) {
+  return attention_strip_shape(head_dim) && n >= 2u && rows <= 16u * kStripMaxGroups &&
+         rows >= attention_strip_rows(head_dim, heads, kv_heads, n, grouped, quantized, token_major);
+}
+
+bool attention_strip_shape(size_t head_dim) { return head_dim == 64u || head_dim == 128u; }
 
 // Groups a kv head has room for in the packed rows, and their floats.
 static uint32_t strip_cap(size_t context) {
@@ -863,6 +888,12 @@ hipError_t launch_rope_append(const float* qr, const float* kr, const float* vr,
 }  // namespace rh
 
 extern "C" {
+
+// Test hook: whether a batch of n tokens whose rows end at `rows` takes strips.
+int rh_strip_route_host(size_t head_dim, size_t heads, size_t kv_heads, size_t rows, size_t n, int grouped,
+                        int quantized, int token_major) {
+  return rh::attention_strip_ok(head_dim, heads, kv_heads, rows, n, grouped, quantized, token_major);
+}
 
 // Test hook: workgroup b's tile and run of heads; returns the grid.
 uint32_t rh_strip_place_host(uint32_t b, uint32_t tiles, uint32_t hx, uint32_t* tile, uint32_t* heads) {

@@ -1355,11 +1355,12 @@ rh_status forward_device(rh_decoder* d, const uint32_t* tokens, size_t n, size_t
   const uint32_t grp = static_cast<uint32_t>(c.head_count / c.head_count_kv);
   const size_t glds = attention_group_lds_floats(grp, start + n) * 4u;
   const bool groupable = hd == 64u && (grp == 4u || grp == 8u) && glds <= kMaxLdsBytes;
-  const bool strip = attention_strip_ok(hd, start + n, n, groupable), grouped = groupable && !strip;
   // when both producers of the residual delta (the O and down matrices) are
   // k-quant GEMMs over Q8_K operands, they store it token-major and the
   // norms read it coalesced
-  const bool tm = (strip || grouped) && d->quant_attn && d->quant_ffn && n >= rh_gemm_min_tokens();
+  const bool may_tm = d->quant_attn && d->quant_ffn && n >= rh_gemm_min_tokens();
+  const bool strip = attention_strip_ok(hd, c.head_count, c.head_count_kv, start + n, n, groupable, d->quant_attn, may_tm);
+  const bool grouped = groupable && !strip, tm = (strip || grouped) && may_tm;
   const AddNorm norm_fn = tm ? add_norm_for<false, true>(w) : add_norm_for(w);
   // a batch whose normed rows feed only k-quant GEMMs gets them as Q8_K
   // straight from the norm kernel
@@ -1796,7 +1797,7 @@ rh_status rh_decoder_new(rh_ctx* ctx, const rh_decoder_config* config, const rh_
        dmalloc(&d->pick_parts, c.vocab_size) == hipSuccess &&
        hipHostMalloc(reinterpret_cast<void**>(&d->host_logits), c.vocab_size * 4, hipHostMallocDefault) == hipSuccess &&
        hipHostMalloc(reinterpret_cast<void**>(&d->host_token), 64, hipHostMallocDefault) == hipSuccess &&
-       (!attention_strip_ok(c.head_dim, 2, 2, false) ||
+       (!attention_strip_shape(c.head_dim) ||
         dmalloc(&d->pack, attention_pack_floats(c.context_length, d->kv)) == hipSuccess) &&
        dmalloc(&d->scores, c.head_count * attention_step_pitch(c.context_length)) == hipSuccess &&
        dmalloc(&d->count, 2) == hipSuccess;

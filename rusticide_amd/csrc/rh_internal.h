@@ -188,10 +188,14 @@ hipError_t launch_gemm_i2s(const GemvJobs& jobs, const Q8Dev& q, size_t tokens, 
 // Causal attention of n tokens at positions start.. over the cached rows
 // (attention.hip): q rotated, token-major; the caches hold rows up to
 // start + n; mixed token-major; pack: attention_pack_floats of scratch, whose
-// contents do not outlive the call's work. attention_strip_ok says which
-// batches it takes (rows = start + n; grouped: attention_group_kernel would
-// take the shape).
-bool attention_strip_ok(size_t head_dim, size_t rows, size_t n, bool grouped);
+// contents do not outlive the call's work. attention_strip_shape says which
+// heads it takes, attention_strip_ok which batches (rows = start + n; grouped:
+// attention_group_kernel would take the shape; quantized: the attention
+// output is wanted as the O matrix's Q8_K operand; token_major: k-quant GEMMs
+// on both sides keep their rows token-major around it).
+bool attention_strip_shape(size_t head_dim);
+bool attention_strip_ok(size_t head_dim, size_t heads, size_t kv_heads, size_t rows, size_t n, bool grouped,
+                        bool quantized, bool token_major);
 size_t attention_pack_floats(size_t context, size_t kv);
 hipError_t launch_attention_strip(const float* q, const float* kcache, const float* vcache, float* pack,
                                   size_t context, uint32_t width, uint32_t kv, uint32_t head_dim, float scale,

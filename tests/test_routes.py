@@ -34,3 +34,54 @@ def test_strips_cover_every_tile_and_never_crowd_one_xcd(tiles, hx):
     for b, _ in work:
         load[b % 8] += 1
     assert max(load) - min(load) <= (1 if tiles < 8 and hx >= 32 else hx), load
+
+
+# us a layer of the strips less the kernels they replaced, beside each shape:
+# (head_dim, heads, kv_heads, rows, tokens, grouped, quantized, token-major)
+SLOWER = [
+    (64, 32, 8, 246, 8, 1, 1, 0),     # +2.1
+    (64, 32, 8, 524, 4, 1, 1, 0),     # +1.6
+    (64, 32, 8, 269, 9, 1, 1, 1),     # +2.1
+    (64, 32, 16, 2, 2, 0, 1, 0),      # +4.6
+    (64, 32, 16, 1010, 8, 0, 1, 0),   # +2.5
+    (64, 32, 32, 400, 2, 0, 1, 0),    # +4.5
+    (64, 32, 32, 1230, 8, 0, 1, 0),   # +2.6
+    (64, 40, 8, 604, 2, 0, 1, 0),     # +3.8
+    (64, 8, 4, 408, 8, 0, 0, 0),      # +2.1
+    (64, 32, 32, 140, 16, 0, 0, 0),   # +3.3
+    (64, 32, 16, 48, 24, 0, 0, 0),    # +4.9
+    (128, 16, 4, 2, 2, 0, 1, 0),      # +3.5
+    (128, 16, 16, 128, 8, 0, 1, 0),   # +0.8
+    (128, 8, 1, 32, 16, 0, 0, 0),     # +5.2
+]
+FASTER = [
+    (64, 32, 4, 320, 2, 1, 1, 0),     # -5.9
+    (64, 32, 8, 1010, 2, 1, 1, 0),    # -8.6
+    (64, 32, 8, 404, 24, 1, 1, 1),    # -6.2
+    (64, 32, 16, 1710, 2, 0, 1, 0),   # -1.6
+    (64, 32, 2, 1210, 4, 0, 1, 0),    # -2.3
+    (64, 32, 16, 9, 9, 0, 1, 1),      # -0.3
+    (64, 32, 32, 250, 32, 0, 0, 0),   # -3.7
+    (64, 32, 4, 2000, 2000, 1, 1, 1),
+    (128, 16, 4, 320, 2, 0, 1, 0),    # -4.5
+    (128, 16, 16, 20, 12, 0, 1, 1),   # -3.5
+    (128, 16, 4, 700, 700, 0, 1, 1),
+]
+
+
+@pytest.mark.parametrize("shape", SLOWER + FASTER)
+def test_batches_take_strips_where_those_measured_faster(shape):
+    L = R.lib()
+    L.rh_strip_route_host.argtypes = [ctypes.c_size_t] * 5 + [ctypes.c_int] * 3
+    assert L.rh_strip_route_host(*shape) == (shape in FASTER)
+
+
+def test_strips_take_no_shape_beyond_their_lds_or_one_token():
+    L = R.lib()
+    L.rh_strip_route_host.argtypes = [ctypes.c_size_t] * 5 + [ctypes.c_int] * 3
+    for head_dim, heads, kv_heads in ((64, 32, 4), (64, 32, 8), (64, 32, 32), (128, 16, 4)):
+        grouped = int(head_dim == 64 and heads // kv_heads in (4, 8))
+        assert L.rh_strip_route_host(head_dim, heads, kv_heads, 2496, 64, grouped, 1, 1)
+        assert not L.rh_strip_route_host(head_dim, heads, kv_heads, 2497, 64, grouped, 1, 1)
+        assert not L.rh_strip_route_host(head_dim, heads, kv_heads, 1000, 1, grouped, 1, 0)
+    assert not L.rh_strip_route_host(96, 8, 2, 1000, 64, 0, 1, 1)
