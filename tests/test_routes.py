@@ -85,3 +85,12 @@ def test_strips_take_no_shape_beyond_their_lds_or_one_token():
         assert not L.rh_strip_route_host(head_dim, heads, kv_heads, 2497, 64, grouped, 1, 1)
         assert not L.rh_strip_route_host(head_dim, heads, kv_heads, 1000, 1, grouped, 1, 0)
     assert not L.rh_strip_route_host(96, 8, 2, 1000, 64, 0, 1, 1)
+
+
+@pytest.mark.parametrize("head_dim,rows,split", [
+    (64, 225, 0), (64, 256, 0), (64, 257, 1), (64, 4480, 1), (64, 4500, 0),  # +1.4 us a layer at 235 rows, -0.1 at 260
+    (128, 1, 1), (128, 4480, 1), (128, 4500, 0), (32, 1000, 0), (96, 1000, 0)])
+def test_one_token_takes_the_split_step_where_it_measured_faster(head_dim, rows, split):
+    L = R.lib()
+    L.rh_step_route_host.argtypes = [ctypes.c_size_t] * 2
+    assert L.rh_step_route_host(head_dim, rows) == split
