@@ -864,12 +864,23 @@ hipError_t launch_attention_strip(const float* q, const float* kcache, const flo
 // every length (-3.1 over the first 200 rows).
 constexpr size_t kStepMinRows64 = 257;
 
+// The most rows whose values and weights step_mix_kernel holds.
+constexpr size_t step_max_rows() {
+  size_t rows = 0;
+  while (step_mix_lds_bytes(rows + 4u) <= kLdsBytes) rows += 4u;
+  return rows;
+}
+constexpr size_t kStepMaxRows = step_max_rows();
+
 bool attention_step_long_ok(size_t head_dim, size_t rows) {
-  return ((head_dim == 64u && rows >= kStepMinRows64) || head_dim == 128u) && rows <= 65536u &&
-         step_mix_lds_bytes(rows) <= kLdsBytes;
+  return ((head_dim == 64u && rows >= kStepMinRows64) || head_dim == 128u) && rows <= kStepMaxRows;
 }
 
-size_t attention_step_pitch(size_t context) { return (context + 63u) & ~size_t{63}; }
+size_t attention_step_pitch(size_t context) { return (std::min(context, kStepMaxRows) + 63u) & ~size_t{63}; }
+
+size_t attention_step_floats(size_t head_dim, size_t heads, size_t context) {
+  return attention_step_long_ok(head_dim, std::min(context, kStepMaxRows)) ? heads * attention_step_pitch(context) : 0u;
+}
 
 hipError_t launch_attention_step_long(const float* qr, const float* kr, const float* vr, const float* rcos,
                                       const float* rsin, float* kcache, float* vcache, uint32_t heads, uint32_t kv,
@@ -904,6 +915,11 @@ int rh_strip_route_host(size_t head_dim, size_t heads, size_t kv_heads, size_t r
 
 // Test hook: whether a token at row `rows` takes the split step.
 int rh_step_route_host(size_t head_dim, size_t rows) { return rh::attention_step_long_ok(head_dim, rows); }
+
+// Test hook: floats of the split step's score scratch.
+size_t rh_step_scratch_host(size_t head_dim, size_t heads, size_t context) {
+  return rh::attention_step_floats(head_dim, heads, context);
+}
 
 // Test hook: workgroup b's tile and run of heads; returns the grid.
 uint32_t rh_strip_place_host(uint32_t b, uint32_t tiles, uint32_t hx, uint32_t* tile, uint32_t* heads) {

@@ -1799,7 +1799,7 @@ rh_status rh_decoder_new(rh_ctx* ctx, const rh_decoder_config* config, const rh_
        hipHostMalloc(reinterpret_cast<void**>(&d->host_token), 64, hipHostMallocDefault) == hipSuccess &&
        (!attention_strip_shape(c.head_dim) ||
         dmalloc(&d->pack, attention_pack_floats(c.context_length, d->kv)) == hipSuccess) &&
-       dmalloc(&d->scores, c.head_count * attention_step_pitch(c.context_length)) == hipSuccess &&
+       dmalloc(&d->scores, attention_step_floats(c.head_dim, c.head_count, c.context_length)) == hipSuccess &&
        dmalloc(&d->count, 2) == hipSuccess;
   if (!ok) {
     rh_decoder_free(d);

@@ -202,8 +202,10 @@ hipError_t launch_attention_strip(const float* q, const float* kcache, const flo
                                   uint32_t start, uint32_t n, float* mixed, hipStream_t s);
 // One token's RoPE, KV append and attention over start + 1 rows, from the raw
 // projections; attention_step_long_ok says which rows it takes. scores holds
-// heads rows of `pitch` floats (attention_step_pitch of the context).
+// attention_step_floats of scratch (0 where no length takes it), heads rows of
+// `pitch` floats, attention_step_pitch of the context.
 bool attention_step_long_ok(size_t head_dim, size_t rows);
+size_t attention_step_floats(size_t head_dim, size_t heads, size_t context);
 size_t attention_step_pitch(size_t context);
 hipError_t launch_attention_step_long(const float* qr, const float* kr, const float* vr, const float* rcos,
                                       const float* rsin, float* kcache, float* vcache, uint32_t heads, uint32_t kv,

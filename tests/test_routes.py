@@ -94,3 +94,14 @@ def test_one_token_takes_the_split_step_where_it_measured_faster(head_dim, rows,
     L = R.lib()
     L.rh_step_route_host.argtypes = [ctypes.c_size_t] * 2
     assert L.rh_step_route_host(head_dim, rows) == split
+
+
+@pytest.mark.parametrize("head_dim,heads,context", [(64, 32, 200), (64, 32, 256), (64, 32, 257), (64, 32, 2048),
+                                                    (64, 32, 4488), (64, 32, 32576), (128, 16, 40), (128, 16, 32576),
+                                                    (2, 4096, 32576), (96, 8, 2048)])
+def test_step_scratch_holds_the_rows_the_split_step_takes_and_no_more(head_dim, heads, context):
+    L = R.lib()
+    L.rh_step_route_host.argtypes = [ctypes.c_size_t] * 2
+    L.rh_step_scratch_host.argtypes, L.rh_step_scratch_host.restype = [ctypes.c_size_t] * 3, ctypes.c_size_t
+    rows = max((r for r in range(1, min(context, 6000) + 1) if L.rh_step_route_host(head_dim, r)), default=0)
+    assert L.rh_step_scratch_host(head_dim, heads, context) == heads * ((rows + 63) // 64 * 64)
