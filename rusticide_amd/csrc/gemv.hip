@@ -1938,6 +1938,24 @@ uint32_t choose_blocks_per_team(uint32_t type_id, uint32_t nb, uint32_t total_ro
   return 4u;
 }
 
+// The tiled dense kernel's LDS for `tokens` activations of `cols` values.
+size_t dense_x_bytes(size_t cols, size_t tokens) { return tokens * ((cols + 3u) & ~size_t{3}) * sizeof(float); }
+
+// Whether 16-byte aligned dense rows take the tiled kernel: where it measured
+// faster than gemv_dense_kernel and its activation takes at most 64 KiB beside
+// the tiles. It brings the activation into LDS before its first weight, which
+// short rows do not repay. One token, us, tiled against the other: 32000 x 256
+// 8.1 : 6.8, 32000 x 384 11.0 : 12.7, 12000 x 384 6.6 : 5.7, 12000 x 512 7.9 :
+// 9.3; 5632 x 512 6.9 : 6.5 (more workgroups of one wave than CUs), 2048 x 768
+// 8.2 : 8.7, 5632 x 1024 11.3 : 17.2. Two tokens and more read each row once,
+// the other once a token: 20000 x 64 5.0 : 4.0 (2 tokens), 5.9 : 5.8 (4), 5632
+// x 128 4.2 : 4.8 (2).
+bool dense_tiled(size_t rows, size_t cols, size_t tokens) {
+  if (dense_x_bytes(cols, tokens) > 64u * 1024u) return false;
+  if (tokens > 1u) return tokens * cols >= 256u;
+  return cols >= 1024u || (cols >= 512u && rows <= 4096u) || (cols >= 384u && rows * cols >= 6000000u);
+}
+
 // One grouped launch. FUSED: the k-quant kernels quantize x themselves
 // (T <= kMaxFusedTokens); otherwise they read the activation q holds.
 template <int T>
@@ -2074,12 +2092,10 @@ hipError_t launch_t(uint32_t type_id, GemvJobs jobs, const Q8Dev& q, const float
     if (per % c == 0u) jobs.j[0].il = static_cast<uint32_t>(__builtin_ctz(c)) + 1u;
   }
   if (type_id == 0u) {
-    // the tiled form wherever the rows are 16-byte aligned (a load past a
-    // row's last value stays within the matrix and its slack) and the
-    // activation takes at most 64 KiB of LDS beside the tiles; a workgroup
-    // of 64 rows when that gives every CU one, of 16 otherwise
-    const size_t xb = static_cast<size_t>(T) * ((nbl + 3u) & ~3u) * sizeof(float);
-    bool tiled = xb <= 64u * 1024u;
+    // a load past a row's last value stays within the matrix and its slack;
+    // a workgroup of 64 rows when that gives every CU one, of 16 otherwise
+    const size_t xb = dense_x_bytes(nbl, T);
+    bool tiled = dense_tiled(total_rows, nbl, T);
     for (uint32_t i = 0; i < jobs.n; i++)
       tiled = tiled && jobs.j[i].stride % 16u == 0 && (reinterpret_cast<uintptr_t>(jobs.j[i].w) & 15u) == 0;
     if (tiled) {
@@ -2486,3 +2502,10 @@ hipError_t launch_dequantize_row(uint32_t type_id, const uint8_t* mat, size_t pi
 }
 
 }  // namespace rh
+
+extern "C" {
+
+// Test hook: whether aligned dense rows take the tiled kernel for a launch's tokens.
+int rh_dense_route_host(size_t rows, size_t cols, size_t tokens) { return rh::dense_tiled(rows, cols, tokens); }
+
+}  // extern "C"

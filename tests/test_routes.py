@@ -105,3 +105,24 @@ def test_step_scratch_holds_the_rows_the_split_step_takes_and_no_more(head_dim, 
     L.rh_step_scratch_host.argtypes, L.rh_step_scratch_host.restype = [ctypes.c_size_t] * 3, ctypes.c_size_t
     rows = max((r for r in range(1, min(context, 6000) + 1) if L.rh_step_route_host(head_dim, r)), default=0)
     assert L.rh_step_scratch_host(head_dim, heads, context) == heads * ((rows + 63) // 64 * 64)
+
+
+# us, the tiled kernel and gemv_dense_kernel
+@pytest.mark.parametrize("rows,cols,tokens,tiled", [
+    (64, 8, 1, 0),         # 2.8, 2.1
+    (32000, 8, 1, 0),      # 4.4, 2.6
+    (32000, 64, 1, 0),     # 4.5, 3.3
+    (20000, 64, 2, 0),     # 5.0, 4.0
+    (32000, 32, 5, 0),     # 6.1, 6.0
+    (20000, 256, 1, 0),    # 7.5, 5.1
+    (12000, 384, 1, 0),    # 6.6, 5.7
+    (5632, 512, 1, 0),     # 6.9, 6.5
+    (5632, 128, 2, 1),     # 4.2, 4.8
+    (2048, 768, 1, 1),     # 8.2, 8.7
+    (32000, 384, 1, 1),    # 11.0, 12.7
+    (12000, 512, 1, 1),    # 7.9, 9.3
+    (32000, 2048, 1, 1), (64, 1024, 1, 1), (64, 16384, 1, 1), (64, 16385, 1, 0), (64, 2048, 8, 1), (64, 2052, 8, 0)])
+def test_dense_rows_take_the_tiled_kernel_where_it_measured_faster(rows, cols, tokens, tiled):
+    L = R.lib()
+    L.rh_dense_route_host.argtypes = [ctypes.c_size_t] * 3
+    assert L.rh_dense_route_host(rows, cols, tokens) == tiled
