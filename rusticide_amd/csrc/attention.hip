@@ -15,6 +15,7 @@
 //   * An output lane's value mix is one chain over the rows: k is the row.
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 
 #include "rh_device.h"
 #include "rh_internal.h"
@@ -117,9 +118,10 @@ __device__ __forceinline__ void load_group(const float* row, uint32_t gi, float 
 // The sum in order from 0.0 of a strip row per half-wave (ordered_sum_wave's
 // method, rh_device.h, with 32 lanes a sum): lane hl holds the run of `mine`
 // groups from group hl * per on, `lanes` lanes hold values, and t is an
-// approximate sum of the lane's run. Every lane of the wave calls it.
+// approximate sum of the lane's run. Every lane of the wave calls it. `rounds`
+// as ordered_sum_wave's, one a half-wave.
 __device__ __forceinline__ float ordered_sum_half(const float* row, uint32_t per, uint32_t mine, uint32_t lanes,
-                                                  uint32_t groups, float t) {
+                                                  uint32_t groups, float t, uint32_t* rounds = nullptr) {
   const uint32_t lane = __lane_id(), hl = lane & 31u, half = lane >> 5;
   const uint32_t g0 = hl * per;
   double d = t;
@@ -174,6 +176,7 @@ __device__ __forceinline__ float ordered_sum_half(const float* row, uint32_t per
 #pragma unroll
         for (int i = 0; i < 16; i++) end += x[i];
       }
+      if (rounds && hl == 0u) rounds[half] = bad_h ? r + 1u : r;
       return end;
     }
     const float start = state == 1u ? cand[1] : state == 2u ? cand[2] : cand[0];
@@ -803,6 +806,78 @@ hipError_t launch_strips(const float* q, const float* kcache, const float* vcach
   return hipSuccess;
 }
 
+// ---- test hooks' kernels, one wave each
+
+// ordered_sum_half over values[0][0..n0) and values[1][0..n1), in strip rows
+// of `stride` floats, +0.0 past their ends as the masked exps are.
+__global__ __launch_bounds__(64) void ordered_sum_half_kernel(const float* values, uint32_t n0, uint32_t n1,
+                                                              uint32_t groups, uint32_t stride, float* out,
+                                                              uint32_t* rounds) {
+  extern __shared__ __align__(16) float sh[];
+  for (uint32_t j = 0; j < 2u; j++)
+    for (uint32_t i = threadIdx.x; i < 16u * groups; i += 64u)
+      sh[j * stride + 4u * strip_slot((i >> 4) * 4u + (i & 3u)) + ((i >> 2) & 3u)] =
+          i < (j ? n1 : n0) ? values[j * 16u * groups + i] : 0.0f;
+  __syncthreads();
+  const uint32_t half = threadIdx.x >> 5, hl = threadIdx.x & 31u, rows = half ? n1 : n0;
+  const float* const row = sh + half * stride;
+  const uint32_t per = (groups + 31u) >> 5, own = (rows + 15u) >> 4, lanes = (own + per - 1u) / per;
+  const uint32_t mine = hl < lanes ? min(per, own - hl * per) : 0u;
+  float t = 0.0f;
+  for (uint32_t c = 0; c < mine; c++) {
+    float x[16];
+    load_group(row, hl * per + c, x);
+    for (int i = 0; i < 16; i++) t += x[i];
+  }
+  const float sum = ordered_sum_half(row, per, mine, lanes, own, t, rounds);
+  if (hl == 0u) out[half] = sum;
+}
+
+// y[i] = x[i] / d by div_by, n a multiple of 4.
+__global__ __launch_bounds__(64) void div_by_kernel(const float* x, uint32_t n, float d, float* y) {
+  const double inv = 1.0 / static_cast<double>(d);
+  for (uint32_t i = blockIdx.x * 64u + threadIdx.x; i < n / 4u; i += 64u * gridDim.x) {
+    f32x4 v = reinterpret_cast<const f32x4*>(x)[i];
+    div_by(v, d, inv);
+    reinterpret_cast<f32x4*>(y)[i] = v;
+  }
+}
+
+// d[16][16] = the MFMA chain over a[16][k] and b[k][16] from 0.0.
+__global__ __launch_bounds__(64) void mfma_chain_kernel(const float* a, const float* b, uint32_t k, float* d) {
+  const uint32_t j = threadIdx.x & 15u, kq = threadIdx.x >> 4;
+  v4f acc{};
+  for (uint32_t s = 0; s < k; s += 4u)
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j * k + s + kq], b[(s + kq) * 16u + j], acc, 0, 0, 0);
+#pragma unroll
+  for (uint32_t i = 0; i < 4u; i++) d[(4u * kq + i) * 16u + j] = acc[i];
+}
+
+constexpr size_t kMaxHookValues = size_t{1} << 24;
+
+// in[0..n) to the device, `launch` on it and m floats of output, those back.
+template <typename Launch>
+rh_status run_hook(rh_ctx* ctx, const float* in, size_t n, float* out, size_t m, Launch launch) {
+  if (hipSetDevice(ctx_device(ctx)) != hipSuccess) return RH_ERR_DEVICE;
+  const hipStream_t s = static_cast<hipStream_t>(rh_stream(ctx));
+  float *din = nullptr, *dout = nullptr;
+  if (hipMalloc(reinterpret_cast<void**>(&din), n * 4u) != hipSuccess) return RH_ERR_OUT_OF_MEMORY;
+  if (hipMalloc(reinterpret_cast<void**>(&dout), m * 4u) != hipSuccess) {
+    (void)hipFree(din);
+    return RH_ERR_OUT_OF_MEMORY;
+  }
+  hipError_t e = hipMemcpyAsync(din, in, n * 4u, hipMemcpyHostToDevice, s);
+  if (e == hipSuccess) {
+    launch(din, dout, s);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess) e = hipMemcpyAsync(out, dout, m * 4u, hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  (void)hipFree(din);
+  (void)hipFree(dout);
+  return e == hipSuccess ? RH_OK : RH_ERR_DEVICE;
+}
+
 }  // namespace
 
 // Rows (cached and new) from which a batch of n tokens takes strips: the
@@ -906,6 +981,43 @@ hipError_t launch_rope_append(const float* qr, const float* kr, const float* vr,
 }  // namespace rh
 
 extern "C" {
+
+// Test hook: the softmax's ordered sums of a strip's two rows, values[0] and
+// values[1] at a distance of whole groups of 16 (16 * groups floats each);
+// rounds: as rh_ordered_sum_device, one a row.
+rh_status rh_ordered_sum_half_device(rh_ctx* ctx, const float* values, size_t groups, size_t n0, size_t n1, float* sums,
+                                     uint32_t* rounds) {
+  if (!ctx || !values || !sums || !rounds || groups == 0 || groups > rh::kStripMaxGroups || n0 == 0 || n1 == 0 ||
+      n0 > 16u * groups || n1 > 16u * groups)
+    return RH_ERR_INVALID_ARGUMENT;
+  float out[4] = {};
+  const uint32_t g = static_cast<uint32_t>(groups), stride = rh::strip_stride(g);
+  const rh_status st = rh::run_hook(ctx, values, 32u * groups, out, 4, [&](float* in, float* o, hipStream_t s) {
+    hipLaunchKernelGGL(rh::ordered_sum_half_kernel, dim3(1), dim3(64), 8u * stride, s, in, static_cast<uint32_t>(n0),
+                       static_cast<uint32_t>(n1), g, stride, o, reinterpret_cast<uint32_t*>(o + 2));
+  });
+  std::memcpy(sums, out, 8);
+  std::memcpy(rounds, out + 2, 8);
+  return st;
+}
+
+// Test hook: x[i] / d as the softmax divides its weights; n a multiple of 4.
+rh_status rh_div_by_device(rh_ctx* ctx, const float* x, size_t n, float d, float* y) {
+  if (!ctx || !x || !y || n == 0 || n % 4u || n > rh::kMaxHookValues) return RH_ERR_INVALID_ARGUMENT;
+  return rh::run_hook(ctx, x, n, y, n, [&](float* in, float* o, hipStream_t s) {
+    hipLaunchKernelGGL(rh::div_by_kernel, dim3(256), dim3(64), 0, s, in, static_cast<uint32_t>(n), d, o);
+  });
+}
+
+// Test hook: the products of a[16][k] and b[k][16] (one after the other at ab)
+// on the f32 matrix cores, as the attention kernels form their chains; k a
+// multiple of 4.
+rh_status rh_mfma_chain_device(rh_ctx* ctx, const float* ab, size_t k, float* d) {
+  if (!ctx || !ab || !d || k == 0 || k % 4u || 32u * k > rh::kMaxHookValues) return RH_ERR_INVALID_ARGUMENT;
+  return rh::run_hook(ctx, ab, 32u * k, d, 256, [&](float* in, float* o, hipStream_t s) {
+    hipLaunchKernelGGL(rh::mfma_chain_kernel, dim3(1), dim3(64), 0, s, in, in + 16u * k, static_cast<uint32_t>(k), o);
+  });
+}
 
 // Test hook: whether a batch of n tokens whose rows end at `rows` takes strips.
 int rh_strip_route_host(size_t head_dim, size_t heads, size_t kv_heads, size_t rows, size_t n, int grouped,

@@ -181,7 +181,8 @@ def test_graph_cache_evicts_within_one_generate_call(ctx, monkeypatch):
 def test_head_dims_other_than_64_take_the_generic_attention(ctx, norm_path, head_dim, heads, kv_heads, width):
     # attention_kernel<0> (any even head_dim up to 128; above 64, 32-row value
     # tiles and a second wave of output lanes) in the batched and the
-    # one-token forwards, against the CPU path
+    # one-token forwards, against the CPU path; head_dim 128 takes it for the
+    # five tokens only, the strips for 64 and the split step for one
     cfg = dict(SMALL, embedding_length=width, head_count=heads, head_count_kv=kv_heads, head_dim=head_dim)
     model = synth.decoder_model(cfg, seed=head_dim)
     gpu, cpu = R.Decoder(ctx, model), O.Decoder(model, threads=8)
