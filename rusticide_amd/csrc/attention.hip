@@ -7,8 +7,9 @@
 // The CPU path's order of float operations fits the f32 MFMA: one
 // v_mfma_f32_16x16x4 adds its four products to the accumulator one fused
 // multiply-add at a time, k ascending, each rounded to nearest with
-// subnormals kept (compared bit for bit with fmaf chains over normal,
-// subnormal, overflowing, signed-zero, infinite and NaN operands).
+// subnormals kept (tests/test_gpu_attention_edges.py compares it bit for bit
+// with fmaf chains over normal, subnormal, overflowing, signed-zero, infinite
+// and NaN operands).
 //   * A score is eight interleaved chains of fused adds (dot's eight lanes),
 //     added in order: chain l is an accumulator of its own, its k the
 //     eight-wide chunks; the eight accumulators are then added in order.
@@ -245,15 +246,16 @@ __host__ __device__ constexpr StripPlace strip_place(uint32_t b, uint32_t tiles,
 //   2. softmax: each half-wave takes one query row: exp, the ordered sum,
 //      the division, in LDS;
 //   3. the value mix: wave w owns output lanes 16w .. of all 16 query rows,
-//      one MFMA per four cached rows, values straight from memory. The groups that reach past some query row's last cached
-//      row are added lane by lane, so that no masked row enters a chain.
+//      one MFMA per four cached rows, values straight from memory. The groups
+//      that reach past some query row's last cached row are added lane by
+//      lane, so that no masked row enters a chain.
 // The scores stay in LDS between the phases (64 bytes a cached row), which
 // caps a launch at kStripMaxGroups groups.
 // What bounds it: the two products' MFMAs, HD / 4 of 32 cycles each a 16 x 16
 // tile on four SIMDs, 13 us of a strip over 2000 rows of 64; measured, the
 // scores take 9.7 us of it, the mix, one chain a SIMD, 11.9, and the softmax
 // between them, which one workgroup a CU cannot overlap, 13.
-// 2000 tokens of 32 heads of 64 over 4 kv heads: 339 us a layer with the
+// 2000 tokens of 32 heads of 64 over 4 kv heads: 339-349 us a layer with the
 // packing, against 2521 for attention_group_kernel (a workgroup a token and
 // kv head); 700 tokens of 16 heads of 128: 50 us against 381 for
 // attention_kernel.
@@ -262,8 +264,9 @@ __host__ __device__ constexpr StripPlace strip_place(uint32_t b, uint32_t tiles,
 template <uint32_t HD, bool ONE>
 __global__ __launch_bounds__(kStripThreads, !ONE && HD == 64u ? 4 : 2) void attention_strip_kernel(
     const float* __restrict__ q, const float* __restrict__ kpack, const float* __restrict__ vpack,
-    const float* __restrict__ vcache, uint32_t cap, uint32_t width, uint32_t kv, uint32_t heads, uint32_t hs_log, uint32_t group, float scale, uint32_t start, uint32_t n,
-    uint32_t tile0, uint32_t tiles, uint32_t stride, float* __restrict__ mixed) {
+    const float* __restrict__ vcache, uint32_t cap, uint32_t width, uint32_t kv, uint32_t heads, uint32_t hs_log,
+    uint32_t group, float scale, uint32_t start, uint32_t n, uint32_t tile0, uint32_t tiles, uint32_t stride,
+    float* __restrict__ mixed) {
   constexpr uint32_t MQ = HD / 32u;   // MFMA steps of a score chain
   constexpr uint32_t DT = HD / 16u;   // output tiles of 16 lanes
   constexpr uint32_t KA = ONE ? 4u : 2u, kMixAhead = ONE ? 16u : 8u;  // groups of keys, of values requested ahead

@@ -10,8 +10,8 @@
 // from int8 MFMA (v_mfma_i32_32x32x32_i8), exact in i32:
 //   * the sub-block scale is folded into the weight and the product split
 //     into two int8 planes: Q4_K w = sc*q with sc = 8*sh + sl, planes sh*q
-//     and sl*q (0..105), isum = 8*hi + lo; Q6_K w = sc*(q-32) = 128*hi + lo
-//     (lo in 0..127, hi in -32..31), isum = 128*hi + lo. Two accumulators
+//     and sl*q (0..105), isum = 8*hi + lo; Q6_K w = sc*(q-32) = 256*hi + lo
+//     (lo in -128..127, hi in -16..16), isum = 256*hi + lo. Two accumulators
 //     take the planes side by side over the block's eight 32-deep steps, so
 //     each activation fragment is read from LDS once for both;
 //   * the Q4_K min term needs only the block sums: with bsum = 128*bh + bl
@@ -320,8 +320,8 @@ __device__ __forceinline__ void lane_planes(const LaneRaw<12>& x, uint32_t kk, u
 // + lo, lo in -128..127). The bytes are spread into 16-bit lanes and multiplied
 // with one packed multiply-add each, which gives w + 128 (|w| <= 4096): its
 // high byte is hi, its low byte less 128 lo, gathered with v_perm_b32. Seven
-// operations where a split at 128 took nine (2048 x 5632 for 509 tokens, bound
-// by this decoding: 50.0 against 52.8 us).
+// operations where a split at 128 took nine (2048 x 5632 for 509 tokens: 50.0
+// against 52.8 us).
 __device__ __forceinline__ void q6_split(uint32_t q, int32_t sc, uint32_t& hi, uint32_t& lo) {
   typedef int16_t i16x2 __attribute__((ext_vector_type(2)));
   const i16x2 scv{static_cast<int16_t>(sc), static_cast<int16_t>(sc)};

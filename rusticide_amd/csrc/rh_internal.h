@@ -107,7 +107,7 @@ struct Tuning {
   int gemm_bn = 0;         // RUSTICIDE_HIP_GEMM_BN=32|64: tokens a GEMM workgroup
   bool gemm_split = true;  // RUSTICIDE_HIP_GEMM_SPLIT=0
   bool gemm_fixup = true;  // RUSTICIDE_HIP_GEMM_FIXUP=0: a split GEMM's planes summed by gemm_combine_kernel
-  bool attn_lds = true;    // RUSTICIDE_HIP_ATTN_LDS=0: the tiled attention step only
+  bool attn_lds = true;    // RUSTICIDE_HIP_ATTN_LDS=0: neither the LDS-staged nor the split step
 };
 const Tuning& tuning();
 void load_tuning();  // publish a fresh snapshot from the environment
